@@ -296,7 +296,9 @@ def main():
                                                         "velocity_error": verr(sol)}
     R = paths[head]
     kname = {"mixed_gmres": "k_sor_colour_f32"}.get(head, "k_sor_colour")
-    if head == "mixed_gmres" and tuning:
+    if head == "mixed_gmres" and args.pc == "multigrid":
+        kname = "k_patch_smooth"        # both smoothings: precond_sweeps sweeps and A z per launch
+    elif head == "mixed_gmres" and tuning:
         kname = f"k_sor_colour_f32_tuned<{tuning['threads_per_block']},{tuning['schedule']},{tuning['loads']}>"
     meets = [k for k, v in ladder.items() if v["velocity_error"] <= 1e-6]
     out = {

@@ -1,0 +1,85 @@
+"""Sweeps on patches (one launch per smoothing, halo rows recomputed by every
+patch that needs them) against the per-colour kernels: the same operations on
+the same values, so the same bits."""
+import os
+
+import numpy as np
+import pytest
+
+from ufemism_amd import abi, batch, geometry
+from ufemism_amd.dynamics import Step, frozen_ssa_system
+
+pytestmark = pytest.mark.gpu
+
+
+def _linear(wl, on, precision, nu):
+    os.environ["UFE_AMG_PATCH"] = on
+    ctx = abi.Context(0)
+    try:
+        frozen_ssa_system(ctx, wl, picard=2)
+        ctx.fill("U_SSA_AaAc", 0.0)
+        ctx.fill("V_SSA_AaAc", 0.0)
+        st = ctx.ssa_linear_solve(1e-8, 100000, precision=precision, gmres=20, precond_sweeps=nu, orth_passes=1,
+                                  precond_type=abi.UFE_PRECOND_MULTIGRID)
+        return st.matvecs, st.sweeps, ctx.get("U_SSA_AaAc"), ctx.get("V_SSA_AaAc")
+    finally:
+        ctx.close()
+        os.environ.pop("UFE_AMG_PATCH", None)
+
+
+@pytest.mark.parametrize("kind,n,nu", [("dome", 300, 2), ("dome", 2000, 1), ("marine", 20000, 2), ("marine", 20000, 1),
+                                       ("marine", 90000, 2)])
+@pytest.mark.parametrize("precision", [abi.UFE_MIXED, abi.UFE_FP64])
+def test_multigrid_smoothing_on_patches_is_bit_identical(kind, n, nu, precision):
+    print(f"[patch] {kind} {n} nu {nu} precision {precision}", flush=True)
+    wl = (geometry.dome if kind == "dome" else geometry.marine)(n, seed=5, picard=2)
+    a, b = (_linear(wl, on, precision, nu) for on in ("0", "1"))
+    assert a[:2] == b[:2], (a[:2], b[:2])
+    assert np.array_equal(a[2], b[2]) and np.array_equal(a[3], b[3])
+    assert np.abs(a[2]).max() > 0
+
+
+def test_multigrid_patches_with_prescribed_rows():
+    """The grounding-line flux holds rows of the smoother fixed."""
+    print("[patch] GL flux", flush=True)
+    wl = geometry.marine(20000, seed=5, picard=3)
+    wl.params.use_analytical_GL_flux = True
+    out = {}
+    for on in ("0", "1"):
+        os.environ["UFE_AMG_PATCH"] = on
+        ctx = abi.Context(0)
+        try:
+            step = Step(ctx, wl)
+            ctx.set_params(wl.params, abi.UFE_MIXED, linear_rel_tol=1e-8, precond_type=abi.UFE_PRECOND_MULTIGRID,
+                           precond_sweeps=2)
+            out[on] = step.run()
+        finally:
+            ctx.close()
+            os.environ.pop("UFE_AMG_PATCH", None)
+    assert out["0"]["sweeps"] == out["1"]["sweeps"]
+    for k in ("U_SSA", "V_SSA", "Ux_SSA_Ac", "Uy_SSA_Ac"):
+        assert np.array_equal(out["0"][k], out["1"][k]), k
+
+
+def test_batch_on_patches_is_bit_identical():
+    print("[patch] batch", flush=True)
+    wls = batch.ensemble(n=4, nv_min=1500, nv_max=6000, seed=7, picard=2)
+    out = {}
+    for on in ("0", "1"):
+        os.environ["UFE_AMG_PATCH"] = on
+        ctx = abi.Context(0)
+        try:
+            b = batch.Batch(ctx, wls)
+            ctx.update_general_ice_model_data()
+            for _ in range(2):          # the second pass replays the captured cycle
+                b.reset()
+                ctx.update_general_ice_model_data()
+                st, rel = ctx.batch_solve_SSA(2, rel_tol=1e-8, gmres_restart=20, precond_sweeps=2,
+                                              precond_type=abi.UFE_PRECOND_MULTIGRID)
+            assert st.status == 0, (st.status, rel)
+            out[on] = (st.cycles, ctx.get("U_SSA"), ctx.get("V_SSA"))
+        finally:
+            ctx.close()
+            os.environ.pop("UFE_AMG_PATCH", None)
+    assert out["0"][0] == out["1"][0]
+    assert np.array_equal(out["0"][1], out["1"][1]) and np.array_equal(out["0"][2], out["1"][2])

@@ -20,9 +20,12 @@
 
 #include "ufe_internal.h"
 #include <hip/hip_ext.h>
+#include <type_traits>
 
 #include "ufe_kernels.inc"
 #include "amg_host.h"
+#include "patch_host.h"
+#include "patch_kernels.inc"
 
 namespace ufe {
 
@@ -151,6 +154,15 @@ struct AmgLevel {
   bool kstep = false;               // solved by two cycles with a GCR(2) combination
 };
 
+// A set of patches on the device (patch_host.h), built on first use per mesh.
+enum PatchKind { PATCH_PRE32 = 0, PATCH_POST32, PATCH_KINDS };
+struct PatchSet {
+  bool built = false, ok = false;   // ok: the mesh fits (otherwise the per-colour kernels run)
+  int bs = 0;                       // threads per workgroup
+  size_t lds = 0;
+  PatchDev P{};
+};
+
 struct ufe_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -178,6 +190,10 @@ struct ufe_ctx {
   // AaAc colour order
   int32_t *d_perm = nullptr, *d_iperm = nullptr;
   std::vector<int32_t> h_perm;
+  std::vector<uint32_t> h_key;      // Hilbert key of each row
+  std::vector<uint16_t> h_mid;      // batch member of each row (empty: single mesh)
+  PatchSet patch[PATCH_KINDS][2];   // by kind and sweeps - 1
+  int32_t *d_place = nullptr;       // 0: SOR row; k: edge point k - 1; -k: corner k - 1
   uint8_t *d_skip = nullptr;        // SOR rows prescribed by the grounding-line flux
   bool gl_active = false;
   int64_t *d_chunk_ptr = nullptr;
@@ -292,6 +308,7 @@ struct ufe_ctx {
   int amg_graph_T_nu = 0;
   double2 *amg_y64 = nullptr;       // FP64 fine-level A z (adjoint)
   float2 *amg_v32 = nullptr, *amg_z32 = nullptr;   // FP32 copies around an FP64 Krylov method
+  float2 *amg_zt = nullptr, *amg_zu = nullptr;     // fine vector between the smoothings (patches)
   double amg_setup_seconds = 0.0;
   int amg_tail_l0 = 0;              // first level solved by k_amg_tail (0: none)
   size_t amg_tail_lds = 0;          // dynamic LDS k_amg_tail may take, bytes
@@ -411,6 +428,12 @@ static void free_mesh(ufe_ctx *ctx) {
   ctx->amg_T = false;
   ctx->amg_y64 = nullptr;
   ctx->amg_v32 = ctx->amg_z32 = nullptr;
+  for (auto &k : ctx->patch)
+    for (PatchSet &S : k) S = PatchSet{};
+  ctx->d_place = nullptr;
+  ctx->h_key.clear();
+  ctx->h_mid.clear();
+  ctx->amg_zt = ctx->amg_zu = nullptr;
 }
 
 static size_t grid_len(const ufe_ctx *ctx, int grid) {
@@ -1609,6 +1632,8 @@ int ufe_mesh_upload(ufe_ctx *ctx, const ufe_mesh_desc *m) try {
   ctx->n_neu = (int)nrow.size();
   ctx->n_cor = (int)crow.size();
   ctx->h_perm = perm;
+  ctx->h_key.resize(nA);
+  for (int p = 0; p < nA; p++) ctx->h_key[p] = (uint32_t)hkey[perm[p]];
   if ((r = dupload(ctx, &ctx->d_perm, perm.data(), nA))) return r;
   if ((r = dupload(ctx, &ctx->d_iperm, iperm.data(), nA))) return r;
   {
@@ -1726,6 +1751,7 @@ int ufe_mesh_upload(ufe_ctx *ctx, const ufe_mesh_desc *m) try {
     }
     ctx->n_chunk = (int)cs.size();
     ctx->h_mch_ptr = mptr;
+    ctx->h_mid = mid;
     if ((r = dupload(ctx, &ctx->d_mid, mid.data(), mid.size()))) return r;
     if ((r = dupload(ctx, &ctx->d_ch_start, cs.data(), cs.size()))) return r;
     if ((r = dupload(ctx, &ctx->d_ch_count, cc.data(), cc.size()))) return r;
@@ -2007,8 +2033,8 @@ static hipEvent_t prof_event(ufe_ctx *ctx) {
 // the dispatch itself (hipExtLaunchKernelGGL), so they time the kernel's own
 // execution and not the queueing around it.
 extern "C++" template <typename K, typename... Args>
-static void timed_kernel(ufe_ctx *ctx, double bytes, int64_t rows, K kernel, dim3 grid, dim3 block,
-                         Args... args) {
+static void timed_kernel_lds(ufe_ctx *ctx, double bytes, int64_t rows, K kernel, dim3 grid, dim3 block, size_t lds,
+                             Args... args) {
   hipEvent_t a = nullptr, b = nullptr;
   // events ride on every PROF_EVERY-th launch: the sample's mean duration is
   // the kernel's, without an event pair on every launch of the timed region
@@ -2023,11 +2049,15 @@ static void timed_kernel(ufe_ctx *ctx, double bytes, int64_t rows, K kernel, dim
     }
   }
   if (!a) {
-    hipLaunchKernelGGL(kernel, grid, block, 0, ctx->stream, args...);
+    hipLaunchKernelGGL(kernel, grid, block, lds, ctx->stream, args...);
     return;
   }
-  hipExtLaunchKernelGGL(kernel, grid, block, 0, ctx->stream, a, b, 0, args...);
+  hipExtLaunchKernelGGL(kernel, grid, block, lds, ctx->stream, a, b, 0, args...);
   ctx->pending.push_back({a, b, bytes, rows});
+}
+extern "C++" template <typename K, typename... Args>
+static void timed_kernel(ufe_ctx *ctx, double bytes, int64_t rows, K kernel, dim3 grid, dim3 block, Args... args) {
+  timed_kernel_lds(ctx, bytes, rows, kernel, grid, block, 0, args...);
 }
 // after a stream synchronisation: fold the recorded pairs into the profile
 static void prof_collect(ufe_ctx *ctx) {
@@ -2807,19 +2837,217 @@ static int amg_capture(ufe_ctx *ctx) {
   return UFE_OK;
 }
 
+// ---------------------------------------------------------------------------
+// Patches (patch_host.h): whole sweeps in one launch
+// ---------------------------------------------------------------------------
+// Own points of a patch and threads of its workgroup.  A thread holds one row
+// of each colour, so the largest colour of the computed rows must fit the
+// workgroup (a patch set that does not fit is built again with 3/4 of the own
+// points).  Larger patches recompute fewer halo rows (1.9 rows per own row at
+// 736, 2.7 at 240); smaller ones fill the 256 CUs on a small mesh.  Measured,
+// own points : threads, on the 1M linear solve / the 182k-vertex batch / the 50k
+// Picard loop / a 30k one (ms; per-colour kernels 67.2 / 56.0 / 71.7 / 24.8):
+// 240:256 69.7 / 52.6 / 59.9 / 19.2, 480:512 64.4 / 51.7 / 55.9 / 19.6, 640:512
+// 60.0 / 49.1 / 55.7 / 19.7, 800:512 57.3 / 48.0 / 54.8 / 19.5, 1000:1024
+// 63.7 / 49.3 / 54.8 / 19.7, 1900:1024 58.0 / 46.9 / 57.1 / 20.1.  736 instead of
+// 800 leaves room for denser colours before the rebuild.
+constexpr size_t PATCH_LDS_MAX = 64 * 1024;
+constexpr int PATCH_LARGE = 1 << 17;   // points from which the large patches fill the chip
+struct PatchShape {
+  int own, bs;
+};
+static PatchShape patch_shape(const ufe_ctx *ctx) {
+  if (ctx->nA >= PATCH_LARGE) return {736, 512};
+  return {std::max(64, std::min(240, ctx->nA / 256)), 256};
+}
+
+// The parts of one patch set in one device allocation
+static int patch_upload(ufe_ctx *ctx, const std::vector<PatchHost> &parts, PatchSet &S, size_t value_bytes) {
+  char *base = nullptr;
+  size_t total = 0;
+  int r;
+  auto put = [&](auto PatchHost::*field, auto *&dst) -> int {
+    using E = typename std::decay_t<decltype(parts[0].*field)>::value_type;
+    size_t n = 0;
+    for (const PatchHost &H : parts) n += (H.*field).size();
+    if (!base) {                     // first round: sizes only
+      total += (n * sizeof(E) + 255) / 256 * 256;
+      return UFE_OK;
+    }
+    E *d = reinterpret_cast<E *>(base + total);
+    dst = d;
+    for (const PatchHost &H : parts) {
+      const auto &v = H.*field;
+      if (!v.empty()) HIPCHK(ctx, hipMemcpyAsync(d, v.data(), v.size() * sizeof(E), hipMemcpyHostToDevice, ctx->stream));
+      d += v.size();
+    }
+    total += (n * sizeof(E) + 255) / 256 * 256;
+    return UFE_OK;
+  };
+  for (int round = 0; round < 2; round++) {
+    if ((r = put(&PatchHost::d, S.P.d)) || (r = put(&PatchHost::rows, S.P.rows)) ||
+        (r = put(&PatchHost::nptr, S.P.nptr)) || (r = put(&PatchHost::sbase, S.P.sbase)) ||
+        (r = put(&PatchHost::lcol, S.P.lcol)) || (r = put(&PatchHost::ov_e, S.P.ov_e)) ||
+        (r = put(&PatchHost::ovf, S.P.ovf)) || (r = put(&PatchHost::ov_c, S.P.ov_c)) ||
+        (r = put(&PatchHost::ncol, S.P.ncol)))
+      return r;
+    if (round == 0) {
+      if ((r = dalloc(ctx, &base, total))) return r;
+      total = 0;
+    }
+  }
+  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));   // the parts go with the caller
+  S.P.np = S.P.cap = S.P.cap_ov = 0;
+  for (const PatchHost &H : parts) {
+    S.P.np += (int)H.d.size();
+    S.P.cap = std::max(S.P.cap, H.max_list);
+    S.P.cap_ov = std::max(S.P.cap_ov, H.max_ov);
+  }
+  S.lds = (size_t)S.P.cap * value_bytes + (size_t)S.P.cap_ov * (value_bytes + sizeof(uint16_t));
+  return UFE_OK;
+}
+
+// Builds the wanted patch sets that are not there yet
+static int patch_prepare(ufe_ctx *ctx, std::initializer_list<PatchKind> kinds, int nu) {
+  bool all = true;
+  for (PatchKind k : kinds) all = all && ctx->patch[k][nu - 1].built;
+  if (all) return UFE_OK;
+  const int nA = ctx->nA, nchunk = (nA + SELL - 1) / SELL;
+  std::vector<int64_t> cptr(nchunk + 1);
+  std::vector<uint8_t> deg(nA);
+  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+  HIPCHK(ctx, hipMemcpy(cptr.data(), ctx->d_chunk_ptr, sizeof(int64_t) * (nchunk + 1), hipMemcpyDeviceToHost));
+  HIPCHK(ctx, hipMemcpy(deg.data(), ctx->d_deg, nA, hipMemcpyDeviceToHost));
+  std::vector<int32_t> col(cptr[nchunk]);
+  HIPCHK(ctx, hipMemcpy(col.data(), ctx->d_col, sizeof(int32_t) * col.size(), hipMemcpyDeviceToHost));
+  auto get = [&](int n, const int32_t *dp, std::vector<int32_t> &h) -> int {
+    h.resize(std::max(n, 1));
+    if (n) HIPCHK(ctx, hipMemcpy(h.data(), dp, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
+    return UFE_OK;
+  };
+  int r;
+  std::vector<int32_t> nr, np, nc, kr, kp, kc;
+  if ((r = get(ctx->n_neu, ctx->d_neu_row, nr)) || (r = get(ctx->n_neu + 1, ctx->d_neu_ptr, np)) ||
+      (r = get(np[ctx->n_neu], ctx->d_neu_col, nc)) || (r = get(ctx->n_cor, ctx->d_cor_row, kr)) ||
+      (r = get(ctx->n_cor + 1, ctx->d_cor_ptr, kp)) || (r = get(kp[ctx->n_cor], ctx->d_cor_col, kc)))
+    return r;
+  const PatchMesh m{nA, ctx->colour_start, ctx->colour_active, cptr.data(), deg.data(), col.data(), ctx->n_neu,
+                    ctx->n_cor, nr.data(), np.data(), nc.data(), kr.data(), kp.data(), kc.data(), ctx->h_key.data(),
+                    ctx->h_mid.empty() ? nullptr : ctx->h_mid.data()};
+  const std::vector<int32_t> order = patch_order(m);
+  if (!ctx->d_place) {
+    std::vector<int32_t> place(nA, 0);
+    for (int i = 0; i < ctx->n_neu; i++) place[nr[i]] = i + 1;
+    for (int i = 0; i < ctx->n_cor; i++) place[kr[i]] = -i - 1;
+    if ((r = dupload(ctx, &ctx->d_place, place.data(), nA))) return r;
+    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+  }
+  for (PatchKind k : kinds) {
+    PatchSet &S = ctx->patch[k][nu - 1];
+    if (S.built) continue;
+    PatchShape sh = patch_shape(ctx);
+    std::vector<PatchHost> parts;
+    const size_t vb = sizeof(float2);
+    bool fits = false;
+    for (int tries = 0; tries < 6 && !fits; tries++, sh.own = sh.own * 3 / 4) {
+      if (!patch_build(m, order, sh.own, nu, k == PATCH_POST32, true, true, parts)) break;
+      fits = true;
+      for (const PatchHost &H : parts)
+        fits = fits && H.max_group <= sh.bs &&
+               (size_t)H.max_list * vb + (size_t)H.max_ov * (vb + sizeof(uint16_t)) <= PATCH_LDS_MAX;
+    }
+    if (fits) {
+      if ((r = patch_upload(ctx, parts, S, vb))) return r;
+      S.bs = sh.bs;
+      S.ok = true;
+    }
+    S.built = true;
+  }
+  return UFE_OK;
+}
+
+// The smoothing of the multigrid cycle runs on patches (one or two sweeps; the
+// per-colour kernels otherwise, or with UFE_AMG_PATCH=0 in the environment when
+// the hierarchy is first used with this sweep count).
+static int amg_patches(ufe_ctx *ctx) {
+  const int nu = std::max(1, ctx->amg_nu);
+  if (nu > 2) return UFE_OK;
+  const char *off = std::getenv("UFE_AMG_PATCH");
+  if (off && off[0] == '0') {
+    for (PatchKind k : {PATCH_PRE32, PATCH_POST32}) ctx->patch[k][nu - 1].built = true;
+    return UFE_OK;
+  }
+  int r;
+  if ((r = patch_prepare(ctx, {PATCH_PRE32, PATCH_POST32}, nu))) return r;
+  if (!ctx->amg_zt) {
+    if ((r = dalloc(ctx, &ctx->amg_zt, (size_t)ctx->nA))) return r;
+    if ((r = dalloc(ctx, &ctx->amg_zu, (size_t)ctx->nA))) return r;
+  }
+  return UFE_OK;
+}
+static bool amg_on_patches(const ufe_ctx *ctx) {
+  const int nu = std::max(1, ctx->amg_nu);
+  return nu <= 2 && ctx->patch[PATCH_PRE32][nu - 1].ok && ctx->patch[PATCH_POST32][nu - 1].ok;
+}
+
+// One smoothing on patches: from zero with the fine residual into y (pre), or
+// from zin with A z into y when y is given (post)
+extern "C++" template <int BS, int NU>
+static void patch_smooth_launch(ufe_ctx *ctx, bool post, float omega, const float2 *v, const float2 *zin, float2 *z,
+                                float2 *y) {
+  const PatchSet &S = ctx->patch[post ? PATCH_POST32 : PATCH_PRE32][NU - 1];
+  const dim3 grid((S.P.np + 7) / 8 * 8), block(BS);
+  const uint8_t *skip = ctx->gl_active ? ctx->d_skip : nullptr;
+  double bytes = 0.0;
+  int64_t rows = 0;
+  for (int c = 0; c < 5; c++) {
+    bytes += NU * ctx->bytes32[c];
+    rows += (int64_t)NU * ctx->colour_active[c];
+  }
+  const float2 *cU = ctx->d_cU32, *EV = ctx->d_EV32;
+  const float *Sxy = ctx->d_Sxy32;
+  if (!post)
+    timed_kernel_lds(ctx, bytes, rows, k_patch_smooth<float, BS, NU, false, true, true, 1>, grid, block, S.lds, S.P, cU,
+                     Sxy, EV, skip, omega, v, zin, z, y);
+  else if (y)
+    timed_kernel_lds(ctx, bytes, rows, k_patch_smooth<float, BS, NU, true, false, true, 2>, grid, block, S.lds, S.P, cU,
+                     Sxy, EV, skip, omega, v, zin, z, y);
+  else
+    timed_kernel_lds(ctx, bytes, rows, k_patch_smooth<float, BS, NU, true, false, true, 0>, grid, block, S.lds, S.P, cU,
+                     Sxy, EV, skip, omega, v, zin, z, y);
+}
+static void patch_smooth(ufe_ctx *ctx, bool post, float omega, const float2 *v, const float2 *zin, float2 *z,
+                         float2 *y) {
+  const int nu = std::max(1, ctx->amg_nu), bs = ctx->patch[post ? PATCH_POST32 : PATCH_PRE32][nu - 1].bs;
+  if (bs == 256) {
+    if (nu == 1) patch_smooth_launch<256, 1>(ctx, post, omega, v, zin, z, y);
+    else patch_smooth_launch<256, 2>(ctx, post, omega, v, zin, z, y);
+  } else {
+    if (nu == 1) patch_smooth_launch<512, 1>(ctx, post, omega, v, zin, z, y);
+    else patch_smooth_launch<512, 2>(ctx, post, omega, v, zin, z, y);
+  }
+}
+
 // z ~ A^-1 v on the fine level: nu forward FP32 SOR sweeps from zero, the
 // coarse correction of the fine residual, nu backward sweeps; z leaves with
 // the Neumann condition on the edge rows, like the SOR preconditioner's.
-static void amg_apply(ufe_ctx *ctx, const AaAcMesh &am, float omega, const float2 *v, float2 *z) {
+// w given: A z as well, when the smoothing computes it (returns whether it did).
+static bool amg_apply(ufe_ctx *ctx, const AaAcMesh &am, float omega, const float2 *v, float2 *z,
+                      float2 *w = nullptr) {
   const int n = ctx->nA, nu = std::max(1, ctx->amg_nu);
-  // the first sweep starts from z = 0 (its first colour pass sets all of z).
-  // The Neumann rows are brought up to date after the last sweep of each
-  // smoothing only: the residual and the output need them, the smoother's own
-  // sweeps converge as well with them one sweep behind (same iteration counts)
-  for (int k = 0; k < nu; k++) enqueue_sweep_fp32(ctx, am, omega, z, v, false, false, k == nu - 1, k == 0);
+  const bool patches = amg_on_patches(ctx);
   AmgLevel &C = ctx->amg[1];
-  k_matvec_residual<<<nblk(n), BLOCK, 0, ctx->stream>>>(am, ctx->d_cU32, ctx->d_Sxy32, ctx->d_EV32,
-                                                       active_ranges(ctx), z, v, ctx->amg_y);
+  if (patches) {
+    patch_smooth(ctx, false, omega, v, nullptr, ctx->amg_zt, ctx->amg_y);
+  } else {
+    // the first sweep starts from z = 0 (its first colour pass sets all of z).
+    // The Neumann rows are brought up to date after the last sweep of each
+    // smoothing only: the residual and the output need them, the smoother's own
+    // sweeps converge as well with them one sweep behind (same iteration counts)
+    for (int k = 0; k < nu; k++) enqueue_sweep_fp32(ctx, am, omega, z, v, false, false, k == nu - 1, k == 0);
+    k_matvec_residual<<<nblk(n), BLOCK, 0, ctx->stream>>>(am, ctx->d_cU32, ctx->d_Sxy32, ctx->d_EV32,
+                                                         active_ranges(ctx), z, v, ctx->amg_y);
+  }
   k_amg_gather<<<nblk(C.n), BLOCK, 0, ctx->stream>>>(C.n, C.mptr, C.mem, ctx->amg_y, nullptr, C.b);
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   (void)hipStreamIsCapturing(ctx->stream, &cap);
@@ -2832,10 +3060,18 @@ static void amg_apply(ufe_ctx *ctx, const AaAcMesh &am, float omega, const float
     if (!launched) (void)hipGetLastError();
   }
   if (!launched) amg_solve_level(ctx, 1);
-  k_amg_prolong<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, C.agg, C.e1, C.e2, C.kstep ? C.sc : nullptr, z,
-                                                   ctx->gl_active ? ctx->d_skip : nullptr);
+  const uint8_t *skip = ctx->gl_active ? ctx->d_skip : nullptr;
+  if (patches) {
+    k_amg_prolong_neumann<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, C.agg, C.e1, C.e2, C.kstep ? C.sc : nullptr,
+                                                             ctx->amg_zt, skip, ctx->amg_zu, neu_list(ctx),
+                                                             cor_list(ctx), ctx->d_place);
+    patch_smooth(ctx, true, omega, v, ctx->amg_zu, z, w);
+    return w != nullptr;
+  }
+  k_amg_prolong<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, C.agg, C.e1, C.e2, C.kstep ? C.sc : nullptr, z, skip);
   neumann_f32(ctx, z);
   for (int k = 0; k < nu; k++) enqueue_sweep_fp32(ctx, am, omega, z, v, true, false, k == nu - 1);
+  return false;
 }
 
 // The same for an FP64 Krylov method: the cycle runs in FP32 on rounded copies
@@ -3303,8 +3539,9 @@ static int gmres_cycle(ufe_ctx *ctx, int m, int ksweeps, double omega, int passe
   }
   for (int j = 0; j < m; j++) {
     T2 *vj = V + (int64_t)j * n, *zj = Z + (int64_t)j * n;
+    bool have_w = false;
     if (ctx->pc_amg) {
-      if (f32) amg_apply(ctx, am, (float)omega, (const float2 *)vj, (float2 *)zj);
+      if (f32) have_w = amg_apply(ctx, am, (float)omega, (const float2 *)vj, (float2 *)zj, (float2 *)w);
       else amg_apply_f64(ctx, am, (float)omega, (const double2 *)vj, (double2 *)zj);
       *cpass += amg_passes(ctx);
     } else {
@@ -3317,7 +3554,9 @@ static int gmres_cycle(ufe_ctx *ctx, int m, int ksweeps, double omega, int passe
       }
       *cpass += precond_passes(ctx, ksweeps);
     }
-    if (f32)
+    if (have_w) {
+      // A z came with the post-smoothing
+    } else if (f32)
       k_matvec<float><<<nb, BLOCK, 0, ctx->stream>>>(am, ctx->d_cU32, ctx->d_Sxy32, ctx->d_EV32, ar, (const float2 *)zj, (float2 *)w);
     else
       k_matvec<double><<<nb, BLOCK, 0, ctx->stream>>>(am, ctx->d_cU, ctx->d_Sxy, ctx->d_pair[1], ar, (const double2 *)zj, (double2 *)w);
@@ -3511,6 +3750,7 @@ int ufe_ssa_linear_solve(ufe_ctx *ctx, const ufe_linsolve_opts *o, ufe_linsolve_
   if (ctx->pc_amg) {
     ctx->amg_T = false;
     if ((r = amg_setup(ctx))) return r;
+    if ((r = amg_patches(ctx))) return r;
     amg_refresh(ctx);
     LAUNCHCHK(ctx);
     if ((r = amg_capture(ctx))) return r;
@@ -4121,8 +4361,9 @@ static void batch_enqueue_cycle(ufe_ctx *ctx, int m, int ks, double omega, doubl
   k_bscale<T, T><<<nb, BLOCK, 0, ctx->stream>>>(n, (const T2 *)ctx->bk_R, ctx->bk_scale, ctx->d_mid, V);
   for (int j = 0; j < m; j++) {
     T2 *vj = V + (int64_t)j * n, *zj = Z + (int64_t)j * n;
+    bool have_w = false;
     if (f32 && ctx->pc_amg) {
-      amg_apply(ctx, am, (float)omega, (const float2 *)vj, (float2 *)zj);
+      have_w = amg_apply(ctx, am, (float)omega, (const float2 *)vj, (float2 *)zj, (float2 *)w);
     } else {
       k_fill<T2><<<nb, BLOCK, 0, ctx->stream>>>(zj, n, T2{T(0), T(0)});
       for (int k = 0; k < ks; k++) {
@@ -4132,7 +4373,9 @@ static void batch_enqueue_cycle(ufe_ctx *ctx, int m, int ks, double omega, doubl
         else enqueue_sweep_fp64_vec(ctx, am, omega, (double2 *)zj, (const double2 *)vj, k & 1, skip, neu);
       }
     }
-    if (f32)
+    if (have_w) {
+      // A z came with the post-smoothing
+    } else if (f32)
       k_matvec<float><<<nb, BLOCK, 0, ctx->stream>>>(am, ctx->d_cU32, ctx->d_Sxy32, ctx->d_EV32, ar,
                                                      (const float2 *)zj, (float2 *)w);
     else
@@ -4226,6 +4469,7 @@ int ufe_batch_linear_solve(ufe_ctx *ctx, const ufe_batch_opts *o, double *member
   if (ctx->pc_amg) {                  // the union of the members as one hierarchy
     ctx->amg_T = false;
     if ((r = amg_setup(ctx))) return r;
+    if ((r = amg_patches(ctx))) return r;
     amg_refresh(ctx);
     LAUNCHCHK(ctx);
     if ((r = amg_capture(ctx))) return r;
