@@ -83,3 +83,58 @@ def test_batch_on_patches_is_bit_identical():
             os.environ.pop("UFE_AMG_PATCH", None)
     assert out["0"][0] == out["1"][0]
     assert np.array_equal(out["0"][1], out["1"][1]) and np.array_equal(out["0"][2], out["1"][2])
+
+
+def _sor_step(wl, on, sweep_batch=0):
+    os.environ["UFE_SOR_PATCH"] = on
+    ctx = abi.Context(0)
+    try:
+        step = Step(ctx, wl, sweep_batch=sweep_batch)
+        a = step.run()
+        step.reset()
+        b = step.run()              # the second solve starts from other counters and buffers
+        assert a["sweeps"] == b["sweeps"] and np.array_equal(a["U_SSA"], b["U_SSA"])
+        return b
+    finally:
+        ctx.close()
+        os.environ.pop("UFE_SOR_PATCH", None)
+
+
+def _same_step(wl, sweep_batch=0):
+    a, b = _sor_step(wl, "0"), _sor_step(wl, "1", sweep_batch)
+    assert a["sweeps"] == b["sweeps"], (a["sweeps"], b["sweeps"])
+    assert a["stats"].status == b["stats"].status and a["stats"].resets == b["stats"].resets
+    assert a["stats"].last_max_residual == b["stats"].last_max_residual
+    for k in ("U_SSA", "V_SSA", "Ux_SSA_Ac", "Uy_SSA_Ac", "Hi", "eta_AaAc"):
+        assert np.array_equal(a[k], b[k]), k
+    return b
+
+
+# sizes on both sides of each workgroup width: few patches, one per CU, and the
+# widths 256, 512 and 1,024
+@pytest.mark.parametrize("kind,n,picard", [("dome", 60, 3), ("dome", 300, 4), ("dome", 2000, 5), ("dome", 8000, 6),
+                                           ("marine", 20000, 6), ("marine", 37000, 3), ("marine", 70000, 2),
+                                           ("marine", 130000, 2)])
+def test_sor_loop_on_patches_is_bit_identical(kind, n, picard):
+    print(f"[sor patch] {kind} {n}", flush=True)
+    wl = (geometry.dome if kind == "dome" else geometry.marine)(n, seed=5, picard=picard)
+    wl.params.SSA_max_residual_UV = 1e-2     # the reference's 2.5 m/yr ends a fine mesh's first solves after one sweep
+    wl.params.SSA_max_inner_loops = 300
+    r = _same_step(wl)
+    assert sum(r["sweeps"]) > picard
+
+
+def test_sor_loop_on_patches_stops_as_the_sweeps_do():
+    """The sweep limit, launches of a few sweeps, and the reset of an unstable solve."""
+    print("[sor patch] limits", flush=True)
+    wl = geometry.marine(12000, seed=5, picard=4)
+    wl.params.SSA_max_residual_UV = 1e-3
+    for limit in (1, 2, 37):
+        wl.params.SSA_max_inner_loops = limit
+        r = _same_step(wl)
+        assert r["sweeps"] == [limit] * r["picard"] and r["stats"].status == 1
+    wl.params.SSA_max_inner_loops = 200
+    _same_step(wl, sweep_batch=7)
+    wl = geometry.marine(12000, seed=5, picard=2)
+    wl.params.use_analytical_GL_flux = True
+    _same_step(wl)

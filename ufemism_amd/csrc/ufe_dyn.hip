@@ -155,7 +155,7 @@ struct AmgLevel {
 };
 
 // A set of patches on the device (patch_host.h), built on first use per mesh.
-enum PatchKind { PATCH_PRE32 = 0, PATCH_POST32, PATCH_KINDS };
+enum PatchKind { PATCH_PRE32 = 0, PATCH_POST32, PATCH_SOR64, PATCH_KINDS };
 struct PatchSet {
   bool built = false, ok = false;   // ok: the mesh fits (otherwise the per-colour kernels run)
   int bs = 0;                       // threads per workgroup
@@ -193,6 +193,9 @@ struct ufe_ctx {
   std::vector<uint32_t> h_key;      // Hilbert key of each row
   std::vector<uint16_t> h_mid;      // batch member of each row (empty: single mesh)
   PatchSet patch[PATCH_KINDS][2];   // by kind and sweeps - 1
+  double2 *sor_w1 = nullptr;        // second buffer of the SOR loop on patches
+  unsigned long long *sor_slots = nullptr;
+  uint32_t sor_epoch = 0;           // sweeps reported in sor_slots so far
   int32_t *d_place = nullptr;       // 0: SOR row; k: edge point k - 1; -k: corner k - 1
   uint8_t *d_skip = nullptr;        // SOR rows prescribed by the grounding-line flux
   bool gl_active = false;
@@ -431,6 +434,8 @@ static void free_mesh(ufe_ctx *ctx) {
   for (auto &k : ctx->patch)
     for (PatchSet &S : k) S = PatchSet{};
   ctx->d_place = nullptr;
+  ctx->sor_w1 = nullptr;
+  ctx->sor_slots = nullptr;
   ctx->h_key.clear();
   ctx->h_mid.clear();
   ctx->amg_zt = ctx->amg_zu = nullptr;
@@ -2852,17 +2857,29 @@ static int amg_capture(ufe_ctx *ctx) {
 // 63.7 / 49.3 / 54.8 / 19.7, 1900:1024 58.0 / 46.9 / 57.1 / 20.1.  736 instead of
 // 800 leaves room for denser colours before the rebuild.
 constexpr size_t PATCH_LDS_MAX = 64 * 1024;
+constexpr size_t SOR_LDS_MAX = 150 * 1024;   // of the 160 KiB of a CU
+constexpr int SOR_PATCH_MIN = 64;            // own points of a workgroup of the SOR loop, at least
+// LDS of a patch kernel: values, slots beyond the sixth, and (rows) the points' indices
+static size_t patch_lds_bytes(int list, int ov, size_t value_bytes, bool rows) {
+  return (size_t)list * value_bytes + (size_t)ov * value_bytes + (size_t)(ov + 1) / 2 * 4 +
+         (rows ? (size_t)list * sizeof(int32_t) : 0);
+}
 constexpr int PATCH_LARGE = 1 << 17;   // points from which the large patches fill the chip
 struct PatchShape {
   int own, bs;
 };
-static PatchShape patch_shape(const ufe_ctx *ctx) {
+static PatchShape patch_shape(const ufe_ctx *ctx, PatchKind k) {
+  if (k == PATCH_SOR64) {            // at most one workgroup per CU; bs by what the own points need
+    const int own = std::max(SOR_PATCH_MIN, (ctx->nA + SOR_PATCHES - 1) / SOR_PATCHES);
+    return {own, own <= 600 ? 256 : own <= 1400 ? 512 : 1024};
+  }
   if (ctx->nA >= PATCH_LARGE) return {736, 512};
   return {std::max(64, std::min(240, ctx->nA / 256)), 256};
 }
 
 // The parts of one patch set in one device allocation
-static int patch_upload(ufe_ctx *ctx, const std::vector<PatchHost> &parts, PatchSet &S, size_t value_bytes) {
+static int patch_upload(ufe_ctx *ctx, const std::vector<PatchHost> &parts, PatchSet &S, size_t value_bytes,
+                        bool rows) {
   char *base = nullptr;
   size_t total = 0;
   int r;
@@ -2903,11 +2920,12 @@ static int patch_upload(ufe_ctx *ctx, const std::vector<PatchHost> &parts, Patch
     S.P.cap = std::max(S.P.cap, H.max_list);
     S.P.cap_ov = std::max(S.P.cap_ov, H.max_ov);
   }
-  S.lds = (size_t)S.P.cap * value_bytes + (size_t)S.P.cap_ov * (value_bytes + sizeof(uint16_t));
+  S.lds = patch_lds_bytes(S.P.cap, S.P.cap_ov, value_bytes, rows);
   return UFE_OK;
 }
 
 // Builds the wanted patch sets that are not there yet
+static bool sor_patch_resident(ufe_ctx *ctx, const PatchSet &S);
 static int patch_prepare(ufe_ctx *ctx, std::initializer_list<PatchKind> kinds, int nu) {
   bool all = true;
   for (PatchKind k : kinds) all = all && ctx->patch[k][nu - 1].built;
@@ -2945,21 +2963,35 @@ static int patch_prepare(ufe_ctx *ctx, std::initializer_list<PatchKind> kinds, i
   for (PatchKind k : kinds) {
     PatchSet &S = ctx->patch[k][nu - 1];
     if (S.built) continue;
-    PatchShape sh = patch_shape(ctx);
+    PatchShape sh = patch_shape(ctx, k);
     std::vector<PatchHost> parts;
-    const size_t vb = sizeof(float2);
+    const bool sor = k == PATCH_SOR64;
+    const size_t vb = sor ? sizeof(double2) : sizeof(float2);
     bool fits = false;
-    for (int tries = 0; tries < 6 && !fits; tries++, sh.own = sh.own * 3 / 4) {
-      if (!patch_build(m, order, sh.own, nu, k == PATCH_POST32, true, true, parts)) break;
-      fits = true;
-      for (const PatchHost &H : parts)
-        fits = fits && H.max_group <= sh.bs &&
-               (size_t)H.max_list * vb + (size_t)H.max_ov * (vb + sizeof(uint16_t)) <= PATCH_LDS_MAX;
+    for (int tries = 0; tries < 6 && !fits; tries++) {
+      if (!patch_build(m, order, sh.own, nu, k == PATCH_POST32, true, !sor, parts)) break;
+      int group = 0, list = 0, ov = 0;
+      for (const PatchHost &H : parts) {
+        group = std::max(group, H.max_group);
+        list = std::max(list, H.max_list);
+        ov = std::max(ov, H.max_ov);
+      }
+      const size_t lds = patch_lds_bytes(list, ov, vb, sor);
+      fits = group <= sh.bs && lds <= (sor ? SOR_LDS_MAX : PATCH_LDS_MAX);
+      if (fits) break;
+      if (!sor) {
+        sh.own = sh.own * 3 / 4;
+      } else if (group <= 1024 && sh.bs < 1024) {   // the number of workgroups is bounded: wider ones instead
+        fits = group <= (sh.bs = group <= 512 ? 512 : 1024) && lds <= SOR_LDS_MAX;
+        break;
+      } else {
+        break;
+      }
     }
     if (fits) {
-      if ((r = patch_upload(ctx, parts, S, vb))) return r;
+      if ((r = patch_upload(ctx, parts, S, vb, sor))) return r;
       S.bs = sh.bs;
-      S.ok = true;
+      S.ok = !sor || sor_patch_resident(ctx, S);
     }
     S.built = true;
   }
@@ -3166,6 +3198,50 @@ static int sor_batch(ufe_ctx *ctx, const AaAcMesh &m, double omega, double tol, 
   return UFE_OK;
 }
 
+// The sweep loop on patches (k_patch_sor): one launch per solve instead of seven
+// per sweep, the same sweeps and bits.  Not used while kernel times are sampled
+// (the sample is per colour launch), on meshes whose patches exceed a workgroup
+// (about 230,000 vertices), or with UFE_SOR_PATCH=0 in the environment when the
+// mesh is first swept.  Returns the set, or null.
+static const PatchSet *sor_patches(ufe_ctx *ctx, int *err) {
+  *err = UFE_OK;
+  if (ctx->prof) return nullptr;
+  PatchSet &S = ctx->patch[PATCH_SOR64][0];
+  if (!S.built) {
+    const char *off = std::getenv("UFE_SOR_PATCH");
+    if (off && off[0] == '0') {
+      S.built = true;
+      return nullptr;
+    }
+    if ((*err = patch_prepare(ctx, {PATCH_SOR64}, 1))) return nullptr;
+    if (S.ok) {
+      if ((*err = dalloc(ctx, &ctx->sor_w1, (size_t)ctx->nA))) return nullptr;
+      if ((*err = dalloc(ctx, &ctx->sor_slots, (size_t)4 * SOR_PATCHES))) return nullptr;
+      k_fill<unsigned long long><<<nblk(4 * SOR_PATCHES), BLOCK, 0, ctx->stream>>>(ctx->sor_slots, 4 * SOR_PATCHES, 0ull);
+      ctx->sor_epoch = 0;
+    }
+  }
+  return S.ok ? &S : nullptr;
+}
+static const void *sor_patch_kernel(int bs) {
+  return bs == 256 ? reinterpret_cast<const void *>(&k_patch_sor<256, false>)
+         : bs == 512 ? reinterpret_cast<const void *>(&k_patch_sor<512, false>)
+                     : reinterpret_cast<const void *>(&k_patch_sor<1024, true>);
+}
+// Whether the device keeps all workgroups of the loop resident
+static bool sor_patch_resident(ufe_ctx *ctx, const PatchSet &S) {
+  int coop = 0, cus = 0, per = 0;
+  const void *k = sor_patch_kernel(S.bs);
+  if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, ctx->device) != hipSuccess || !coop ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess ||
+      hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S.lds) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k, S.bs, S.lds) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return S.P.np <= SOR_PATCHES && (S.P.np + 7) / 8 * 8 <= per * cus;
+}
+
 static int run_sor_reference(ufe_ctx *ctx, double tol, int max_sweeps, SorFlags *out, double *seconds) {
   const AaAcMesh m = aaac_mesh(ctx);
   const double omega = ctx->params.SSA_SOR_omega;
@@ -3174,6 +3250,35 @@ static int run_sor_reference(ufe_ctx *ctx, double tol, int max_sweeps, SorFlags 
   int batch = ctx->params.sweep_batch > 0 ? ctx->params.sweep_batch : 1;
   int queued = 0;
   auto t0 = std::chrono::steady_clock::now();
+  int perr;
+  if (const PatchSet *S = max_sweeps > 0 ? sor_patches(ctx, &perr) : (perr = UFE_OK, nullptr)) {
+    // a launch holds the device for its sweeps, so a long solve takes several
+    int limit = ctx->params.sweep_batch > 0 ? ctx->params.sweep_batch : 1024, swept = 0, top = max_sweeps;
+    PatchDev P = S->P;
+    const double2 *cU = ctx->d_cU, *EV = ctx->d_pair[1], *RHS = ctx->d_pair[2];
+    const double *Sxy = ctx->d_Sxy;
+    const uint8_t *skip = ctx->gl_active ? ctx->d_skip : nullptr;
+    double om = omega, tl = tol;
+    double2 *W0 = ctx->d_pair[0], *W1 = ctx->sor_w1;
+    unsigned long long *slots = ctx->sor_slots;
+    SorFlags *fl = ctx->d_flags;
+    while (true) {
+      uint32_t epoch = ctx->sor_epoch;
+      void *args[] = {&P, &cU, &Sxy, &EV, &RHS, &skip, &om, &tl, &top, &limit, &W0, &W1, &slots, &epoch, &fl};
+      HIPCHK(ctx, hipLaunchCooperativeKernel(sor_patch_kernel(S->bs), dim3((P.np + 7) / 8 * 8), dim3(S->bs), args,
+                                             (unsigned)S->lds, ctx->stream));
+      HIPCHK(ctx, hipMemcpyAsync(ctx->h_flags, ctx->d_flags, sizeof(SorFlags), hipMemcpyDeviceToHost, ctx->stream));
+      HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+      ctx->sor_epoch += (uint32_t)(ctx->h_flags->sweep - swept);
+      swept = ctx->h_flags->sweep;
+      if (ctx->h_flags->done || swept >= max_sweeps) break;
+    }
+    if (seconds) *seconds += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+    *out = *ctx->h_flags;
+    return UFE_OK;
+  } else if (perr) {
+    return perr;
+  }
   while (true) {
     const int nb = std::min(batch, max_sweeps - queued);
     int r;
