@@ -73,6 +73,25 @@ extern "C" long check(int nA, const int *cs, const int *ca, const int64_t *cptr,
     }
   std::vector<PatchHost> parts;
   if (!patch_build(m, order, own, nu, backward != 0, neumann != 0, ring != 0, parts)) return -2;
+  // the points that patches exchange between sweeps, marked in a copy
+  {
+    std::vector<PatchHost> shared = parts;
+    patch_mark_shared(nA, shared);
+    std::vector<char> read(nA, 0), marked(nA, 0);
+    size_t list0 = 0;
+    for (size_t q = 0; q < parts.size(); q++) {
+      for (const PatchDesc &d : parts[q].d)
+        for (int i = 0; i < d.nlist; i++) {
+          const int32_t p = parts[q].rows[d.list - list0 + i], s = shared[q].rows[d.list - list0 + i];
+          if ((s & 0x7fffffff) != p) return -11;
+          if (i >= d.ncs + d.ne + d.nk) read[p] = 1;
+          if (s < 0) marked[p]++;
+        }
+      list0 += parts[q].rows.size();
+    }
+    for (int p = 0; p < nA; p++)
+      if (read[p] != marked[p]) return -12;
+  }
   PatchHost H;
   auto join = [](auto &a, auto &b) { a.insert(a.end(), b.begin(), b.end()); };
   for (PatchHost &q : parts) {
@@ -179,7 +198,7 @@ def lib(tmp_path_factory):
     d = tmp_path_factory.mktemp("patch")
     (d / "check.cpp").write_text(DRIVER)
     so = d / "check.so"
-    subprocess.run([cxx, "-std=c++17", "-O2", "-ffp-contract=off", "-Wall", "-fPIC", "-shared", "-pthread", f"-I{CSRC}",
+    subprocess.run([cxx, "-std=c++17", "-O2", "-ffp-contract=off", "-Wall", "-Wextra", "-Wno-unused-parameter", "-fPIC", "-shared", "-pthread", f"-I{CSRC}",
                     str(d / "check.cpp"), "-o", str(so)], check=True)
     return ctypes.CDLL(str(so))
 

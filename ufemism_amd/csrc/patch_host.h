@@ -54,7 +54,7 @@ struct PatchHost {                // a part of the patches, one after another
   std::vector<int32_t> rows, nptr;
   std::vector<uint32_t> sbase, lcol, ov_e;   // sbase: SELL position of the first slot, degree in the top 5 bits
   std::vector<uint16_t> ovf, ov_c, ncol;
-  int max_list = 0, max_group = 0, max_ov = 0;
+  int max_list = 0, max_group = 0, max_ov = 0, max_ncs = 0, max_neu = 0, max_ncol = 0;
 };
 
 constexpr int PATCH_BASE_BITS = 27;
@@ -294,6 +294,9 @@ inline bool patch_build(const PatchMesh &m, const std::vector<int32_t> &order, i
       }
       H.max_list = std::max(H.max_list, n);
       H.max_ov = std::max(H.max_ov, D.nov);
+      H.max_ncs = std::max(H.max_ncs, D.ncs);
+      H.max_neu = std::max(H.max_neu, D.ne + D.nk);
+      if (neumann) H.max_ncol = std::max(H.max_ncol, H.nptr.back() - H.nptr[D.nptr]);
       H.d.push_back(D);
     }
     std::free(where);
@@ -317,6 +320,31 @@ inline bool patch_build(const PatchMesh &m, const std::vector<int32_t> &order, i
     ncol += H.ncol.size();
   }
   return 3 * comp < (size_t)INT32_MAX && list < (size_t)INT32_MAX;
+}
+
+// Marks (by the sign bit of rows) the own points that another patch reads
+// without computing them: the values the patches exchange between sweeps.
+inline void patch_mark_shared(int nA, std::vector<PatchHost> &part) {
+  std::vector<uint8_t> read(nA, 0);
+  auto each = [&](auto f) {
+    size_t list0 = 0;                // rows before this part
+    for (PatchHost &H : part) {
+      for (const PatchDesc &d : H.d) f(H.rows.data() + (d.list - list0), d);
+      list0 += H.rows.size();
+    }
+  };
+  each([&](int32_t *rows, const PatchDesc &d) {
+    for (int i = d.ncs + d.ne + d.nk; i < d.nlist; i++) read[rows[i]] = 1;
+  });
+  each([&](int32_t *rows, const PatchDesc &d) {
+    auto mark = [&](int first, int n) {
+      for (int i = first; i < first + n; i++)
+        if (read[rows[i]]) rows[i] |= INT32_MIN;
+    };
+    for (int c = 0; c < 5; c++) mark(d.g[c], d.own[c]);
+    mark(d.ncs, d.own_e);
+    mark(d.ncs + d.ne, d.own_k);
+  });
 }
 
 }  // namespace ufe

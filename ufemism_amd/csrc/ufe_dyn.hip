@@ -194,8 +194,8 @@ struct ufe_ctx {
   std::vector<uint16_t> h_mid;      // batch member of each row (empty: single mesh)
   PatchSet patch[PATCH_KINDS][2];   // by kind and sweeps - 1
   double2 *sor_w1 = nullptr;        // second buffer of the SOR loop on patches
-  unsigned long long *sor_slots = nullptr;
-  uint32_t sor_epoch = 0;           // sweeps reported in sor_slots so far
+  uint32_t *sor_reports = nullptr;
+  uint32_t sor_epoch = 0;           // sweeps reported in sor_reports so far
   int32_t *d_place = nullptr;       // 0: SOR row; k: edge point k - 1; -k: corner k - 1
   uint8_t *d_skip = nullptr;        // SOR rows prescribed by the grounding-line flux
   bool gl_active = false;
@@ -435,7 +435,7 @@ static void free_mesh(ufe_ctx *ctx) {
     for (PatchSet &S : k) S = PatchSet{};
   ctx->d_place = nullptr;
   ctx->sor_w1 = nullptr;
-  ctx->sor_slots = nullptr;
+  ctx->sor_reports = nullptr;
   ctx->h_key.clear();
   ctx->h_mid.clear();
   ctx->amg_zt = ctx->amg_zu = nullptr;
@@ -2857,29 +2857,31 @@ static int amg_capture(ufe_ctx *ctx) {
 // 63.7 / 49.3 / 54.8 / 19.7, 1900:1024 58.0 / 46.9 / 57.1 / 20.1.  736 instead of
 // 800 leaves room for denser colours before the rebuild.
 constexpr size_t PATCH_LDS_MAX = 64 * 1024;
-constexpr size_t SOR_LDS_MAX = 150 * 1024;   // of the 160 KiB of a CU
+constexpr size_t SOR_LDS_MAX = 156 * 1024;   // of the 160 KiB of a CU
 constexpr int SOR_PATCH_MIN = 64;            // own points of a workgroup of the SOR loop, at least
-// LDS of a patch kernel: values, slots beyond the sixth, and (rows) the points' indices
-static size_t patch_lds_bytes(int list, int ov, size_t value_bytes, bool rows) {
-  return (size_t)list * value_bytes + (size_t)ov * value_bytes + (size_t)(ov + 1) / 2 * 4 +
-         (rows ? (size_t)list * sizeof(int32_t) : 0);
+constexpr int PATCH_CUS = 256;               // CUs of an MI355X
+constexpr int PATCH_LARGE = 1 << 17;         // points from which the large patches fill the chip
+// LDS of a smoothing: values, coefficients and columns of the slots beyond the sixth
+static size_t patch_lds_bytes(int list, int ov) {
+  return (size_t)list * sizeof(float2) + (size_t)ov * (sizeof(float2) + sizeof(uint16_t));
 }
-constexpr int PATCH_LARGE = 1 << 17;   // points from which the large patches fill the chip
 struct PatchShape {
   int own, bs;
 };
 static PatchShape patch_shape(const ufe_ctx *ctx, PatchKind k) {
-  if (k == PATCH_SOR64) {            // at most one workgroup per CU; bs by what the own points need
+  if (k == PATCH_SOR64) {            // at most one workgroup per CU; its width follows from the rows
     const int own = std::max(SOR_PATCH_MIN, (ctx->nA + SOR_PATCHES - 1) / SOR_PATCHES);
-    return {own, own <= 600 ? 256 : own <= 1400 ? 512 : 1024};
+    return {own, 0};
   }
-  if (ctx->nA >= PATCH_LARGE) return {736, 512};
+  if (ctx->nA >= PATCH_LARGE) {
+    const int one = (ctx->nA + PATCH_CUS - 1) / PATCH_CUS;   // a workgroup for each CU
+    return {one <= 800 ? one : 736, 512};
+  }
   return {std::max(64, std::min(240, ctx->nA / 256)), 256};
 }
 
 // The parts of one patch set in one device allocation
-static int patch_upload(ufe_ctx *ctx, const std::vector<PatchHost> &parts, PatchSet &S, size_t value_bytes,
-                        bool rows) {
+static int patch_upload(ufe_ctx *ctx, const std::vector<PatchHost> &parts, PatchSet &S) {
   char *base = nullptr;
   size_t total = 0;
   int r;
@@ -2914,13 +2916,6 @@ static int patch_upload(ufe_ctx *ctx, const std::vector<PatchHost> &parts, Patch
     }
   }
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));   // the parts go with the caller
-  S.P.np = S.P.cap = S.P.cap_ov = 0;
-  for (const PatchHost &H : parts) {
-    S.P.np += (int)H.d.size();
-    S.P.cap = std::max(S.P.cap, H.max_list);
-    S.P.cap_ov = std::max(S.P.cap_ov, H.max_ov);
-  }
-  S.lds = patch_lds_bytes(S.P.cap, S.P.cap_ov, value_bytes, rows);
   return UFE_OK;
 }
 
@@ -2966,30 +2961,32 @@ static int patch_prepare(ufe_ctx *ctx, std::initializer_list<PatchKind> kinds, i
     PatchShape sh = patch_shape(ctx, k);
     std::vector<PatchHost> parts;
     const bool sor = k == PATCH_SOR64;
-    const size_t vb = sor ? sizeof(double2) : sizeof(float2);
     bool fits = false;
-    for (int tries = 0; tries < 6 && !fits; tries++) {
+    for (int tries = 0; tries < 6 && !fits; tries++, sh.own = sh.own * 3 / 4) {
       if (!patch_build(m, order, sh.own, nu, k == PATCH_POST32, true, !sor, parts)) break;
-      int group = 0, list = 0, ov = 0;
+      int group = 0;
+      S.P = PatchDev{};
       for (const PatchHost &H : parts) {
         group = std::max(group, H.max_group);
-        list = std::max(list, H.max_list);
-        ov = std::max(ov, H.max_ov);
+        S.P.np += (int)H.d.size();
+        S.P.cap = std::max(S.P.cap, H.max_list);
+        S.P.cap_ov = std::max(S.P.cap_ov, H.max_ov);
+        S.P.cap_ncs = std::max(S.P.cap_ncs, H.max_ncs);
+        S.P.cap_neu = std::max(S.P.cap_neu, H.max_neu);
+        S.P.cap_ncol = std::max(S.P.cap_ncol, H.max_ncol);
       }
-      const size_t lds = patch_lds_bytes(list, ov, vb, sor);
-      fits = group <= sh.bs && lds <= (sor ? SOR_LDS_MAX : PATCH_LDS_MAX);
-      if (fits) break;
-      if (!sor) {
-        sh.own = sh.own * 3 / 4;
-      } else if (group <= 1024 && sh.bs < 1024) {   // the number of workgroups is bounded: wider ones instead
-        fits = group <= (sh.bs = group <= 512 ? 512 : 1024) && lds <= SOR_LDS_MAX;
-        break;
-      } else {
+      if (sor) {                       // the number of workgroups is bounded: wide enough ones or none
+        sh.bs = group <= 256 ? 256 : group <= 512 ? 512 : 1024;
+        S.lds = patch_sor_lds(S.P, sh.bs == 1024);
+        fits = group <= 1024 && S.lds <= SOR_LDS_MAX;
         break;
       }
+      S.lds = patch_lds_bytes(S.P.cap, S.P.cap_ov);
+      fits = group <= sh.bs && S.lds <= PATCH_LDS_MAX;
     }
     if (fits) {
-      if ((r = patch_upload(ctx, parts, S, vb, sor))) return r;
+      if (sor) patch_mark_shared(nA, parts);
+      if ((r = patch_upload(ctx, parts, S))) return r;
       S.bs = sh.bs;
       S.ok = !sor || sor_patch_resident(ctx, S);
     }
@@ -3024,7 +3021,7 @@ static bool amg_on_patches(const ufe_ctx *ctx) {
 
 // One smoothing on patches: from zero with the fine residual into y (pre), or
 // from zin with A z into y when y is given (post)
-extern "C++" template <int BS, int NU>
+extern "C++" template <int BS, int WAVES, int NU>
 static void patch_smooth_launch(ufe_ctx *ctx, bool post, float omega, const float2 *v, const float2 *zin, float2 *z,
                                 float2 *y) {
   const PatchSet &S = ctx->patch[post ? PATCH_POST32 : PATCH_PRE32][NU - 1];
@@ -3039,25 +3036,26 @@ static void patch_smooth_launch(ufe_ctx *ctx, bool post, float omega, const floa
   const float2 *cU = ctx->d_cU32, *EV = ctx->d_EV32;
   const float *Sxy = ctx->d_Sxy32;
   if (!post)
-    timed_kernel_lds(ctx, bytes, rows, k_patch_smooth<float, BS, NU, false, true, true, 1>, grid, block, S.lds, S.P, cU,
+    timed_kernel_lds(ctx, bytes, rows, k_patch_smooth<float, BS, WAVES, NU, false, true, true, 1>, grid, block, S.lds, S.P, cU,
                      Sxy, EV, skip, omega, v, zin, z, y);
   else if (y)
-    timed_kernel_lds(ctx, bytes, rows, k_patch_smooth<float, BS, NU, true, false, true, 2>, grid, block, S.lds, S.P, cU,
+    timed_kernel_lds(ctx, bytes, rows, k_patch_smooth<float, BS, WAVES, NU, true, false, true, 2>, grid, block, S.lds, S.P, cU,
                      Sxy, EV, skip, omega, v, zin, z, y);
   else
-    timed_kernel_lds(ctx, bytes, rows, k_patch_smooth<float, BS, NU, true, false, true, 0>, grid, block, S.lds, S.P, cU,
+    timed_kernel_lds(ctx, bytes, rows, k_patch_smooth<float, BS, WAVES, NU, true, false, true, 0>, grid, block, S.lds, S.P, cU,
                      Sxy, EV, skip, omega, v, zin, z, y);
 }
 static void patch_smooth(ufe_ctx *ctx, bool post, float omega, const float2 *v, const float2 *zin, float2 *z,
                          float2 *y) {
-  const int nu = std::max(1, ctx->amg_nu), bs = ctx->patch[post ? PATCH_POST32 : PATCH_PRE32][nu - 1].bs;
-  if (bs == 256) {
-    if (nu == 1) patch_smooth_launch<256, 1>(ctx, post, omega, v, zin, z, y);
-    else patch_smooth_launch<256, 2>(ctx, post, omega, v, zin, z, y);
-  } else {
-    if (nu == 1) patch_smooth_launch<512, 1>(ctx, post, omega, v, zin, z, y);
-    else patch_smooth_launch<512, 2>(ctx, post, omega, v, zin, z, y);
-  }
+  const int nu = std::max(1, ctx->amg_nu);
+  const PatchSet &S = ctx->patch[post ? PATCH_POST32 : PATCH_PRE32][nu - 1];
+  auto go = [&](auto one, auto two) {
+    if (nu == 1) one(ctx, post, omega, v, zin, z, y);
+    else two(ctx, post, omega, v, zin, z, y);
+  };
+  if (S.bs == 256) go(patch_smooth_launch<256, 2, 1>, patch_smooth_launch<256, 2, 2>);
+  else if (S.P.np <= PATCH_CUS) go(patch_smooth_launch<512, 2, 1>, patch_smooth_launch<512, 2, 2>);
+  else go(patch_smooth_launch<512, 4, 1>, patch_smooth_launch<512, 4, 2>);
 }
 
 // z ~ A^-1 v on the fine level: nu forward FP32 SOR sweeps from zero, the
@@ -3216,8 +3214,8 @@ static const PatchSet *sor_patches(ufe_ctx *ctx, int *err) {
     if ((*err = patch_prepare(ctx, {PATCH_SOR64}, 1))) return nullptr;
     if (S.ok) {
       if ((*err = dalloc(ctx, &ctx->sor_w1, (size_t)ctx->nA))) return nullptr;
-      if ((*err = dalloc(ctx, &ctx->sor_slots, (size_t)4 * SOR_PATCHES))) return nullptr;
-      k_fill<unsigned long long><<<nblk(4 * SOR_PATCHES), BLOCK, 0, ctx->stream>>>(ctx->sor_slots, 4 * SOR_PATCHES, 0ull);
+      if ((*err = dalloc(ctx, &ctx->sor_reports, (size_t)SOR_REPORT_WORDS))) return nullptr;
+      k_fill<uint32_t><<<nblk(SOR_REPORT_WORDS), BLOCK, 0, ctx->stream>>>(ctx->sor_reports, SOR_REPORT_WORDS, 0u);
       ctx->sor_epoch = 0;
     }
   }
@@ -3259,12 +3257,13 @@ static int run_sor_reference(ufe_ctx *ctx, double tol, int max_sweeps, SorFlags 
     const double *Sxy = ctx->d_Sxy;
     const uint8_t *skip = ctx->gl_active ? ctx->d_skip : nullptr;
     double om = omega, tl = tol;
+    int nA = ctx->nA;
     double2 *W0 = ctx->d_pair[0], *W1 = ctx->sor_w1;
-    unsigned long long *slots = ctx->sor_slots;
+    uint32_t *reports = ctx->sor_reports;
     SorFlags *fl = ctx->d_flags;
     while (true) {
       uint32_t epoch = ctx->sor_epoch;
-      void *args[] = {&P, &cU, &Sxy, &EV, &RHS, &skip, &om, &tl, &top, &limit, &W0, &W1, &slots, &epoch, &fl};
+      void *args[] = {&P, &cU, &Sxy, &EV, &RHS, &skip, &om, &tl, &top, &limit, &nA, &W0, &W1, &reports, &epoch, &fl};
       HIPCHK(ctx, hipLaunchCooperativeKernel(sor_patch_kernel(S->bs), dim3((P.np + 7) / 8 * 8), dim3(S->bs), args,
                                              (unsigned)S->lds, ctx->stream));
       HIPCHK(ctx, hipMemcpyAsync(ctx->h_flags, ctx->d_flags, sizeof(SorFlags), hipMemcpyDeviceToHost, ctx->stream));
