@@ -3261,20 +3261,34 @@ static int run_sor_reference(ufe_ctx *ctx, double tol, int max_sweeps, SorFlags 
     double2 *W0 = ctx->d_pair[0], *W1 = ctx->sor_w1;
     uint32_t *reports = ctx->sor_reports;
     SorFlags *fl = ctx->d_flags;
+    bool refused = false;
     while (true) {
       uint32_t epoch = ctx->sor_epoch;
       void *args[] = {&P, &cU, &Sxy, &EV, &RHS, &skip, &om, &tl, &top, &limit, &nA, &W0, &W1, &reports, &epoch, &fl};
-      HIPCHK(ctx, hipLaunchCooperativeKernel(sor_patch_kernel(S->bs), dim3((P.np + 7) / 8 * 8), dim3(S->bs), args,
-                                             (unsigned)S->lds, ctx->stream));
+      const hipError_t launch = hipLaunchCooperativeKernel(sor_patch_kernel(S->bs), dim3((P.np + 7) / 8 * 8),
+                                                           dim3(S->bs), args, (unsigned)S->lds, ctx->stream);
+      // the HIP runtime may refuse cooperative launches that the device's
+      // attributes offer (seen in a host program without torch, on the runtime
+      // of ROCm 7.2: hipErrorIllegalState); nothing has run, so the colour
+      // launches take over, for this mesh from here on
+      refused = launch != hipSuccess && swept == 0;
+      if (refused) {
+        (void)hipGetLastError();
+        ctx->patch[PATCH_SOR64][0].ok = false;
+        break;
+      }
+      HIPCHK(ctx, launch);
       HIPCHK(ctx, hipMemcpyAsync(ctx->h_flags, ctx->d_flags, sizeof(SorFlags), hipMemcpyDeviceToHost, ctx->stream));
       HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
       ctx->sor_epoch += (uint32_t)(ctx->h_flags->sweep - swept);
       swept = ctx->h_flags->sweep;
       if (ctx->h_flags->done || swept >= max_sweeps) break;
     }
-    if (seconds) *seconds += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-    *out = *ctx->h_flags;
-    return UFE_OK;
+    if (!refused) {
+      if (seconds) *seconds += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+      *out = *ctx->h_flags;
+      return UFE_OK;
+    }
   } else if (perr) {
     return perr;
   }
