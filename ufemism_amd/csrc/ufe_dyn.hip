@@ -183,6 +183,8 @@ struct ufe_ctx {
   bool rm_ready = false;
   int rm_nVs = 0, rm_nVd = 0, rm_n = 0;
   int32_t *d_rm_nn = nullptr, *d_rm_tvi = nullptr, *d_rm_st = nullptr, *d_rm_en = nullptr, *d_rm_vi = nullptr;
+  double *rm_work = nullptr;         // source derivatives of a second-order remapping (not in allocs: it grows)
+  size_t rm_work_len = 0;
   double *d_rm_tw = nullptr, *d_rm_w0 = nullptr, *d_rm_w1x = nullptr, *d_rm_w1y = nullptr;
   int32_t *d_icount = nullptr;       // small device counters (upwind misses)
   int32_t *d_Aci = nullptr, *d_edgeAc = nullptr, *d_slot_i = nullptr, *d_slot_j = nullptr;
@@ -359,6 +361,10 @@ static inline int nblk(int64_t n, int b = BLOCK) { return (int)((n + b - 1) / b)
 constexpr int PROF_EVERY = 8;     // colour launches per timed sample
 // grid for XCD-major kernels: a multiple of the 8 XCDs
 static inline int xcd_grid(int64_t n) { return (nblk(n) + 7) / 8 * 8; }
+// grid of a layered kernel: points, groups of LAYERS layers, fields
+static inline dim3 layer_grid(int64_t n, int nz, int fields = 1) {
+  return dim3(xcd_grid(n), std::min((nz + LAYERS - 1) / LAYERS, 65535), fields);
+}
 
 template <typename T>
 static int dalloc(ufe_ctx *ctx, T **p, size_t n) {
@@ -386,6 +392,9 @@ static void free_mesh(ufe_ctx *ctx) {
   ctx->d_NxTri = ctx->d_NyTri = ctx->d_R = ctx->d_crit = nullptr;
   ctx->rm_ready = false;
   ctx->rm_nVs = ctx->rm_nVd = ctx->rm_n = 0;
+  if (ctx->rm_work) (void)hipFree(ctx->rm_work);
+  ctx->rm_work = nullptr;
+  ctx->rm_work_len = 0;
   ctx->d_rm_nn = ctx->d_rm_tvi = ctx->d_rm_st = ctx->d_rm_en = ctx->d_rm_vi = nullptr;
   ctx->d_rm_tw = ctx->d_rm_w0 = ctx->d_rm_w1x = ctx->d_rm_w1y = nullptr;
   // work spaces live in allocs too: forget them with the mesh
@@ -1188,7 +1197,7 @@ int ufe_remap_build(ufe_ctx *dst, ufe_ctx *src, const ufe_mesh_geometry_desc *gs
   HIPCHK(dst, s.alloc((void **)&dd, sizeof(double) * nVd));
   k_fill<double><<<nblk(nVs), BLOCK, 0, q>>>(ones, nVs, 1.0);
   k_deriv_Aa<<<nblk(nVs), BLOCK, 0, q>>>(aa_mesh(src), ones, dx, dy);
-  k_rm_apply_cons<<<nblk(nVd), BLOCK, 0, q>>>(nVd, nVs, 1, dst->d_rm_st, dst->d_rm_en, dst->d_rm_vi, dst->d_rm_w0,
+  k_rm_apply_cons<true><<<layer_grid(nVd, 1), BLOCK, 0, q>>>(nVd, nVs, 1, dst->d_rm_st, dst->d_rm_en, dst->d_rm_vi, dst->d_rm_w0,
                                               dst->d_rm_w1x, dst->d_rm_w1y, ones, dx, dy, dd);
   LAUNCHCHK(dst);
   std::vector<double> hd(nVd);
@@ -1276,29 +1285,35 @@ int ufe_remap_field(ufe_ctx *dst, ufe_ctx *src, int method, const double *d_src,
   hipStream_t q = dst->stream;
   HIPCHK(dst, hipStreamSynchronize(src->stream));
   const int nVs = dst->rm_nVs, nVd = dst->rm_nVd;
-  const int64_t nd = (int64_t)nVd * nz;
-  ScratchDev s;
   switch (method) {
     case UFE_REMAP_TRILIN:
-      k_rm_apply_trilin<<<nblk(nd), BLOCK, 0, q>>>(nVd, nVs, nz, dst->d_rm_tvi, dst->d_rm_tw, d_src, d_dst);
+      k_rm_apply_trilin<<<layer_grid(nVd, nz), BLOCK, 0, q>>>(nVd, nVs, nz, dst->d_rm_tvi, dst->d_rm_tw, d_src, d_dst);
       break;
     case UFE_REMAP_NEAREST_NEIGHBOUR:
-      k_rm_apply_nn<<<nblk(nd), BLOCK, 0, q>>>(nVd, nVs, nz, dst->d_rm_nn, d_src, d_dst);
+      k_rm_apply_nn<<<layer_grid(nVd, nz), BLOCK, 0, q>>>(nVd, nVs, nz, dst->d_rm_nn, d_src, d_dst);
       break;
     case UFE_REMAP_CONS_1ST_ORDER:
-      k_rm_apply_cons<<<nblk(nd), BLOCK, 0, q>>>(nVd, nVs, nz, dst->d_rm_st, dst->d_rm_en, dst->d_rm_vi, dst->d_rm_w0,
-                                                 dst->d_rm_w1x, dst->d_rm_w1y, d_src, nullptr, nullptr, d_dst);
+      k_rm_apply_cons<false><<<layer_grid(nVd, nz), BLOCK, 0, q>>>(nVd, nVs, nz, dst->d_rm_st, dst->d_rm_en, dst->d_rm_vi,
+                                                                   dst->d_rm_w0, nullptr, nullptr, d_src, nullptr,
+                                                                   nullptr, d_dst);
       break;
     case UFE_REMAP_CONS_2ND_ORDER: {
-      double *dx, *dy;
-      HIPCHK(dst, s.alloc((void **)&dx, sizeof(double) * (size_t)nVs * nz));
-      HIPCHK(dst, s.alloc((void **)&dy, sizeof(double) * (size_t)nVs * nz));
-      k_deriv_Aa_3D<<<nblk((int64_t)nVs * nz), BLOCK, 0, q>>>(aa_mesh(src), nz, d_src, dx, dy);
-      k_rm_apply_cons<<<nblk(nd), BLOCK, 0, q>>>(nVd, nVs, nz, dst->d_rm_st, dst->d_rm_en, dst->d_rm_vi, dst->d_rm_w0,
-                                                 dst->d_rm_w1x, dst->d_rm_w1y, d_src, dx, dy, d_dst);
-      LAUNCHCHK(dst);
-      HIPCHK(dst, hipStreamSynchronize(q));
-      return UFE_OK;
+      // the derivatives' space is kept until the mesh goes (allocating and
+      // freeing it took longer than the whole remapping)
+      const size_t need = 2 * (size_t)nVs * nz;
+      if (dst->rm_work_len < need) {
+        if (dst->rm_work) HIPCHK(dst, hipFree(dst->rm_work));
+        dst->rm_work = nullptr;
+        dst->rm_work_len = 0;
+        HIPCHK(dst, hipMalloc((void **)&dst->rm_work, sizeof(double) * need));
+        dst->rm_work_len = need;
+      }
+      double *dx = dst->rm_work, *dy = dx + (size_t)nVs * nz;
+      k_deriv_Aa_3D<<<layer_grid(nVs, nz), BLOCK, 0, q>>>(aa_mesh(src), nz, d_src, dx, dy);
+      k_rm_apply_cons<true><<<layer_grid(nVd, nz), BLOCK, 0, q>>>(nVd, nVs, nz, dst->d_rm_st, dst->d_rm_en, dst->d_rm_vi,
+                                                                  dst->d_rm_w0, dst->d_rm_w1x, dst->d_rm_w1y, d_src, dx,
+                                                                  dy, d_dst);
+      break;
     }
     default:
       dst->err = "ufe_remap_field: unknown method";
@@ -1895,9 +1910,8 @@ int ufe_update_general_ice_model_data(ufe_ctx *ctx) {
     return UFE_BAD_INPUT;
   }
   GenFields f = gen_fields(ctx);
-  k_gen_aa1<<<nblk(ctx->nV), BLOCK, 0, ctx->stream>>>(ctx->nV, f);
-  k_gen_ac<<<nblk(ctx->nAc), BLOCK, 0, ctx->stream>>>(ac_mesh(ctx), f);
-  k_gen_aa2<<<nblk(ctx->nV), BLOCK, 0, ctx->stream>>>(aa_mesh(ctx), f);
+  k_gen_ac<<<xcd_grid(ctx->nAc), BLOCK, 0, ctx->stream>>>(ac_mesh(ctx), f);
+  k_gen_aa<<<xcd_grid(ctx->nV), BLOCK, 0, ctx->stream>>>(aa_mesh(ctx), f);
   LAUNCHCHK(ctx);
   // ice_physical_properties closes the routine (src/general_ice_model_data_module.f90:91)
   if (mode != UFE_PHYS_INPUT) {
@@ -1930,20 +1944,30 @@ int ufe_solve_SIA(ufe_ctx *ctx) {
     p.zeta[k] = ctx->params.zeta[k];
     p.zeta_n[k] = std::pow(ctx->params.zeta[k], N_FLOW);
   }
-  k_sia<<<nblk(ctx->nAc), BLOCK, 0, ctx->stream>>>(
-      ctx->nAc, p, F(ctx, "Hi_Ac"), F(ctx, "dHs_dx_Ac"), F(ctx, "dHs_dy_Ac"), F(ctx, "dHs_dp_Ac"),
-      F(ctx, "dHs_do_Ac"), FI(ctx, "mask_sheet_Ac"), F(ctx, "A_flow_Ac"), F(ctx, "D_SIA_3D_Ac"),
-      F(ctx, "D_SIA_Ac"), F(ctx, "Ux_SIA_Ac"), F(ctx, "Uy_SIA_Ac"), F(ctx, "Up_SIA_Ac"), F(ctx, "Uo_SIA_Ac"));
-  AaMesh am = aa_mesh(ctx);
-  k_map_Ac_to_Aa<<<nblk(ctx->nV), BLOCK, 0, ctx->stream>>>(am, ctx->nAc, 1, F(ctx, "Ux_SIA_Ac"), F(ctx, "U_SIA"));
-  k_map_Ac_to_Aa<<<nblk(ctx->nV), BLOCK, 0, ctx->stream>>>(am, ctx->nAc, 1, F(ctx, "Uy_SIA_Ac"), F(ctx, "V_SIA"));
-  k_map_Ac_to_Aa<<<nblk(ctx->nV), BLOCK, 0, ctx->stream>>>(am, ctx->nAc, 1, F(ctx, "D_SIA_Ac"), F(ctx, "D_SIA"));
+  auto sia = [&](auto kernel) {
+    kernel<<<nblk(ctx->nAc), BLOCK, 0, ctx->stream>>>(
+        ctx->nAc, p, F(ctx, "Hi_Ac"), F(ctx, "dHs_dx_Ac"), F(ctx, "dHs_dy_Ac"), F(ctx, "dHs_dp_Ac"),
+        F(ctx, "dHs_do_Ac"), FI(ctx, "mask_sheet_Ac"), F(ctx, "A_flow_Ac"), F(ctx, "D_SIA_3D_Ac"),
+        F(ctx, "D_SIA_Ac"), F(ctx, "Ux_SIA_Ac"), F(ctx, "Uy_SIA_Ac"), F(ctx, "Up_SIA_Ac"), F(ctx, "Uo_SIA_Ac"));
+  };
+  if (p.nZ <= COLUMN_REGS) sia(k_sia<COLUMN_REGS>);
+  else sia(k_sia<MAX_NZ>);
+  k_map3_Ac_to_Aa<<<xcd_grid(ctx->nV), BLOCK, 0, ctx->stream>>>(aa_mesh(ctx), F(ctx, "Ux_SIA_Ac"), F(ctx, "Uy_SIA_Ac"),
+                                                               F(ctx, "D_SIA_Ac"), F(ctx, "U_SIA"), F(ctx, "V_SIA"),
+                                                               F(ctx, "D_SIA"));
   LAUNCHCHK(ctx);
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   return UFE_OK;
 }
 
 // ---- solve_SIA_3D and the critical time steps ---------------------------------
+// apply_Neumann_boundary_3D of one or two fields
+static void neumann_Aa(ufe_ctx *ctx, int nz, double *d0, double *d1 = nullptr) {
+  const int fields = d1 ? 2 : 1;
+  k_neumann_Aa_edges<<<layer_grid(ctx->nV, nz, fields), BLOCK, 0, ctx->stream>>>(aa_mesh(ctx), nz, d0, d1);
+  k_neumann_Aa_corners<<<dim3(nblk(nz, 64), fields), 64, 0, ctx->stream>>>(aa_mesh(ctx), nz, d0, d1);
+}
+
 int ufe_solve_SIA_3D(ufe_ctx *ctx) {
   if (!ctx || !ctx->have_mesh) return UFE_BAD_INPUT;
   SIA3DParams p;
@@ -1971,14 +1995,11 @@ int ufe_solve_SIA_3D(ufe_ctx *ctx) {
   const AaMesh am = aa_mesh(ctx);
   const int nz = ctx->nZ;
   hipStream_t q = ctx->stream;
-  k_sia3d_uv<<<nblk(ctx->nV), BLOCK, 0, q>>>(ctx->nV, p, f);
-  for (double *d : {f.U3, f.V3}) {   // apply_Neumann_boundary_3D (:366-367)
-    k_neumann_Aa_edges<<<nblk((int64_t)ctx->nV * nz), BLOCK, 0, q>>>(am, nz, d);
-    k_neumann_Aa_corners<<<nblk(nz, 64), 64, 0, q>>>(am, nz, d);
-  }
-  k_sia3d_w<<<nblk(ctx->nV), BLOCK, 0, q>>>(am, p, f);
-  k_neumann_Aa_edges<<<nblk((int64_t)ctx->nV * nz), BLOCK, 0, q>>>(am, nz, f.W3);
-  k_neumann_Aa_corners<<<nblk(nz, 64), 64, 0, q>>>(am, nz, f.W3);
+  if (nz <= COLUMN_REGS) k_sia3d_uv<COLUMN_REGS><<<nblk(ctx->nV), BLOCK, 0, q>>>(ctx->nV, p, f);
+  else k_sia3d_uv<MAX_NZ><<<nblk(ctx->nV), BLOCK, 0, q>>>(ctx->nV, p, f);
+  neumann_Aa(ctx, nz, f.U3, f.V3);   // apply_Neumann_boundary_3D (:366-367)
+  k_sia3d_w<<<xcd_grid(ctx->nV), BLOCK, 0, q>>>(am, p, f);
+  neumann_Aa(ctx, nz, f.W3);
   LAUNCHCHK(ctx);
   HIPCHK(ctx, hipStreamSynchronize(q));
   return UFE_OK;
@@ -4827,15 +4848,14 @@ int ufe_op_curvatures_Aa(ufe_ctx *ctx, const double *d, double *a, double *b, do
 }
 int ufe_op_derivatives_Aa_3D(ufe_ctx *ctx, const double *d, double *ddx, double *ddy, int nz) {
   NEED_MESH(ctx);
-  k_deriv_Aa_3D<<<nblk((int64_t)ctx->nV * nz), BLOCK, 0, ctx->stream>>>(aa_mesh(ctx), nz, d, ddx, ddy);
+  k_deriv_Aa_3D<<<layer_grid(ctx->nV, nz), BLOCK, 0, ctx->stream>>>(aa_mesh(ctx), nz, d, ddx, ddy);
   LAUNCHCHK(ctx);
   return ufe_synchronize(ctx);
 }
 int ufe_op_neumann_Aa(ufe_ctx *ctx, double *d) { return ufe_op_neumann_Aa_3D(ctx, d, 1); }
 int ufe_op_neumann_Aa_3D(ufe_ctx *ctx, double *d, int nz) {
   NEED_MESH(ctx);
-  k_neumann_Aa_edges<<<nblk((int64_t)ctx->nV * nz), BLOCK, 0, ctx->stream>>>(aa_mesh(ctx), nz, d);
-  k_neumann_Aa_corners<<<nblk(nz, 64), 64, 0, ctx->stream>>>(aa_mesh(ctx), nz, d);
+  neumann_Aa(ctx, nz, d);
   LAUNCHCHK(ctx);
   return ufe_synchronize(ctx);
 }
@@ -4845,7 +4865,7 @@ int ufe_op_upwind_derivatives_3D(ufe_ctx *ctx, const double *U, const double *V,
   if (!U || !V || !d || !ddx || !ddy || nz < 1) return UFE_BAD_INPUT;
   hipStream_t q = ctx->stream;
   HIPCHK(ctx, hipMemsetAsync(ctx->d_icount, 0, sizeof(int32_t), q));
-  k_upwind_3D<<<nblk((int64_t)ctx->nV * nz), BLOCK, 0, q>>>(aa_mesh(ctx), tri_mesh(ctx), nz, U, V, d, ddx, ddy,
+  k_upwind_3D<<<layer_grid(ctx->nV, nz), BLOCK, 0, q>>>(aa_mesh(ctx), tri_mesh(ctx), nz, U, V, d, ddx, ddy,
                                                             ctx->d_icount);
   LAUNCHCHK(ctx);
   int32_t h = 0;
@@ -4894,14 +4914,14 @@ int ufe_op_neumann_AaAc(ufe_ctx *ctx, double *d) {
 int ufe_op_map_Aa_to_Ac(ufe_ctx *ctx, const double *a, double *b) { return ufe_op_map_Aa_to_Ac_3D(ctx, a, b, 1); }
 int ufe_op_map_Aa_to_Ac_3D(ufe_ctx *ctx, const double *a, double *b, int nz) {
   NEED_MESH(ctx);
-  k_map_Aa_to_Ac<<<nblk((int64_t)ctx->nAc * nz), BLOCK, 0, ctx->stream>>>(ac_mesh(ctx), nz, a, b);
+  k_map_Aa_to_Ac<<<layer_grid(ctx->nAc, nz), BLOCK, 0, ctx->stream>>>(ac_mesh(ctx), nz, a, b);
   LAUNCHCHK(ctx);
   return ufe_synchronize(ctx);
 }
 int ufe_op_map_Ac_to_Aa(ufe_ctx *ctx, const double *a, double *b) { return ufe_op_map_Ac_to_Aa_3D(ctx, a, b, 1); }
 int ufe_op_map_Ac_to_Aa_3D(ufe_ctx *ctx, const double *a, double *b, int nz) {
   NEED_MESH(ctx);
-  k_map_Ac_to_Aa<<<nblk((int64_t)ctx->nV * nz), BLOCK, 0, ctx->stream>>>(aa_mesh(ctx), ctx->nAc, nz, a, b);
+  k_map_Ac_to_Aa<<<layer_grid(ctx->nV, nz), BLOCK, 0, ctx->stream>>>(aa_mesh(ctx), ctx->nAc, nz, a, b);
   LAUNCHCHK(ctx);
   return ufe_synchronize(ctx);
 }
