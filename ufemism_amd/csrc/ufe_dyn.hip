@@ -312,6 +312,8 @@ struct ufe_ctx {
   hipGraphExec_t amg_graph_T = nullptr;
   int amg_graph_T_nu = 0;
   double2 *amg_y64 = nullptr;       // FP64 fine-level A z (adjoint)
+  double2 *amg_zt64 = nullptr;      // fine vector between the transposed smoothings (patches)
+  bool cor_apart = false;           // no two corners average the same point, none another corner
   float2 *amg_v32 = nullptr, *amg_z32 = nullptr;   // FP32 copies around an FP64 Krylov method
   float2 *amg_zt = nullptr, *amg_zu = nullptr;     // fine vector between the smoothings (patches)
   double amg_setup_seconds = 0.0;
@@ -438,7 +440,8 @@ static void free_mesh(ufe_ctx *ctx) {
   ctx->amg_graph_T = nullptr;
   ctx->amg_graph_T_nu = 0;
   ctx->amg_T = false;
-  ctx->amg_y64 = nullptr;
+  ctx->amg_y64 = ctx->amg_zt64 = nullptr;
+  ctx->cor_apart = false;
   ctx->amg_v32 = ctx->amg_z32 = nullptr;
   for (auto &k : ctx->patch)
     for (PatchSet &S : k) S = PatchSet{};
@@ -2973,6 +2976,10 @@ static int patch_prepare(ufe_ctx *ctx, std::initializer_list<PatchKind> kinds, i
     std::vector<int32_t> place(nA, 0);
     for (int i = 0; i < ctx->n_neu; i++) place[nr[i]] = i + 1;
     for (int i = 0; i < ctx->n_cor; i++) place[kr[i]] = -i - 1;
+    std::vector<int32_t> met(kr.begin(), kr.begin() + ctx->n_cor);
+    met.insert(met.end(), kc.begin(), kc.begin() + kp[ctx->n_cor]);
+    std::sort(met.begin(), met.end());
+    ctx->cor_apart = std::adjacent_find(met.begin(), met.end()) == met.end();
     if ((r = dupload(ctx, &ctx->d_place, place.data(), nA))) return r;
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   }
@@ -3135,26 +3142,83 @@ static void amg_apply_f64(ufe_ctx *ctx, const AaAcMesh &am, float omega, const d
 
 static void apply_AT(ufe_ctx *ctx, const AaAcMesh &mT, const ActiveRanges &ar, const double2 *x, double2 *y,
                      bool keep_fixed = false);
+static void fold_T(ufe_ctx *ctx, double2 *y);
+static RevList rev_list(ufe_ctx *c);
+
+// The transposed smoothings run on the patches of the FP32 smoothing: A^T has the
+// same neighbour lists (its zero couplings to edge points read points that stay
+// zero), and the rows of the Neumann halo are computed along with the others.
+static size_t patch_lds_bytes64(const PatchDev &P) {
+  return (size_t)P.cap * sizeof(double2) + (size_t)P.cap_ov * (sizeof(double2) + sizeof(uint16_t));
+}
+static bool amg_T_on_patches(const ufe_ctx *ctx) {
+  if (!amg_on_patches(ctx) || !ctx->amg_zt64) return false;
+  const int nu = std::max(1, ctx->amg_nu);
+  return patch_lds_bytes64(ctx->patch[PATCH_PRE32][nu - 1].P) <= PATCH_LDS_MAX &&
+         patch_lds_bytes64(ctx->patch[PATCH_POST32][nu - 1].P) <= PATCH_LDS_MAX;
+}
+extern "C++" template <int BS, int NU>
+static void patch_smooth_T_launch(ufe_ctx *ctx, const AaAcMesh &mT, bool post, double omega, const double2 *v,
+                                  const double2 *zin, double2 *z, double2 *y) {
+  const PatchSet &S = ctx->patch[post ? PATCH_POST32 : PATCH_PRE32][NU - 1];
+  const dim3 grid((S.P.np + 7) / 8 * 8), block(BS);
+  const uint8_t *skip = ctx->gl_active ? ctx->d_skip : nullptr;
+  const size_t lds = patch_lds_bytes64(S.P);
+  if (!post)
+    k_patch_smooth<double, BS, 2, NU, false, true, false, 2><<<grid, block, lds, ctx->stream>>>(
+        S.P, mT.cU, mT.Sxy, ctx->d_pair[1], skip, omega, v, zin, z, y);
+  else
+    k_patch_smooth<double, BS, 2, NU, true, false, false, 2><<<grid, block, lds, ctx->stream>>>(
+        S.P, mT.cU, mT.Sxy, ctx->d_pair[1], skip, omega, v, zin, z, y);
+}
+// nu transposed sweeps from zero (forward) or from zin (post, backward) into z,
+// and y = P^T A^T R^T z
+static void patch_smooth_T(ufe_ctx *ctx, const AaAcMesh &mT, bool post, double omega, const double2 *v,
+                           const double2 *zin, double2 *z, double2 *y) {
+  const int nu = std::max(1, ctx->amg_nu);
+  const bool narrow = ctx->patch[post ? PATCH_POST32 : PATCH_PRE32][nu - 1].bs == 256;
+  auto go = narrow ? (nu == 1 ? patch_smooth_T_launch<256, 1> : patch_smooth_T_launch<256, 2>)
+                   : (nu == 1 ? patch_smooth_T_launch<512, 1> : patch_smooth_T_launch<512, 2>);
+  go(ctx, mT, post, omega, v, zin, z, y);
+  const uint8_t *skip = ctx->gl_active ? ctx->d_skip : nullptr;
+  const NeumannList E = neu_list(ctx), K = cor_list(ctx);
+  if (E.n + K.n <= FOLD_MAX) {
+    k_fold_T<<<1, FOLD_THREADS, 0, ctx->stream>>>(mT, E, K, rev_list(ctx), skip, z, y, ctx->cor_apart ? 1 : 0);
+    return;
+  }
+  k_edge_rows_T<<<nblk(E.n + K.n), BLOCK, 0, ctx->stream>>>(mT, E, K, z, y);
+  fold_T(ctx, y);
+  if (skip) k_zero_skip_rows<<<nblk(ctx->nA), BLOCK, 0, ctx->stream>>>(ctx->nA, skip, y);
+}
 
 // The transposed operator P^T A^T R^T of the adjoint solves: nu forward FP64
 // transposed SOR sweeps from zero (edge rows stay zero), the coarse correction
 // on the transposed hierarchy (ctx->amg_T set by the caller), nu backward
-// sweeps.
-static void amg_apply_T(ufe_ctx *ctx, const AaAcMesh &mT, double omega, const double2 *v, double2 *z) {
+// sweeps, and w = P^T A^T R^T z.
+// On patches a smoothing with its operator product is 2 launches and reads the
+// coefficients once; on colours it is 14 (40k vertices: 161 -> 66 us).
+static void amg_apply_T(ufe_ctx *ctx, const AaAcMesh &mT, double omega, const double2 *v, double2 *z, double2 *w) {
   const int n = ctx->nA, nu = std::max(1, ctx->amg_nu);
+  const bool patches = amg_T_on_patches(ctx);
+  const uint8_t *skip = ctx->gl_active ? ctx->d_skip : nullptr;
+  double2 *zt = patches ? ctx->amg_zt64 : z;   // between the smoothings
   auto sweep = [&](bool backward) {
     for (int i = 0; i < 5; i++) {
       const int c = backward ? 4 - i : i;
       const int m = ctx->colour_active[c];
       if (m == 0) continue;
       k_sor_colour<<<xcd_grid(m), BLOCK, 0, ctx->stream>>>(mT, z, ctx->d_pair[1], v, ctx->colour_start[c], m,
-                                                         omega, nullptr, ctx->gl_active ? ctx->d_skip : nullptr);
+                                                         omega, nullptr, skip);
     }
   };
-  k_fill<double2><<<nblk(n), BLOCK, 0, ctx->stream>>>(z, n, make_double2(0.0, 0.0));
-  for (int k = 0; k < nu; k++) sweep(false);
   AmgLevel &C = ctx->amg[1];
-  apply_AT(ctx, mT, active_ranges(ctx), z, ctx->amg_y64);
+  if (patches) {
+    patch_smooth_T(ctx, mT, false, omega, v, nullptr, zt, ctx->amg_y64);
+  } else {
+    k_fill<double2><<<nblk(n), BLOCK, 0, ctx->stream>>>(z, n, make_double2(0.0, 0.0));
+    for (int k = 0; k < nu; k++) sweep(false);
+    apply_AT(ctx, mT, active_ranges(ctx), z, ctx->amg_y64);
+  }
   k_amg_gather64<<<nblk(C.n), BLOCK, 0, ctx->stream>>>(C.n, C.mptr, C.mem, v, ctx->amg_y64, C.b);
   bool launched = false;
   if (ctx->amg_graph_T) {
@@ -3162,9 +3226,13 @@ static void amg_apply_T(ufe_ctx *ctx, const AaAcMesh &mT, double omega, const do
     if (!launched) (void)hipGetLastError();
   }
   if (!launched) amg_solve_level(ctx, 1);   // the same kernels, eager
-  k_amg_prolong64<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, C.agg, C.e1, C.e2, C.kstep ? C.sc : nullptr, z,
-                                                     ctx->gl_active ? ctx->d_skip : nullptr);
+  k_amg_prolong64<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, C.agg, C.e1, C.e2, C.kstep ? C.sc : nullptr, zt, skip);
+  if (patches) {
+    patch_smooth_T(ctx, mT, true, omega, v, zt, z, w);
+    return;
+  }
   for (int k = 0; k < nu; k++) sweep(true);
+  apply_AT(ctx, mT, active_ranges(ctx), z, w);
 }
 
 // colour passes of one multigrid application (for the sweep count)
@@ -4158,8 +4226,10 @@ static int adj_solve(ufe_ctx *ctx, double tol, int m, int ks, double omega, int 
     int r;
     ctx->amg_T = false;
     if ((r = amg_setup(ctx))) return r;
-    ctx->amg_T = true;
     ctx->amg_nu = ks;
+    if ((r = amg_patches(ctx))) return r;
+    if (amg_on_patches(ctx) && !ctx->amg_zt64 && (r = dalloc(ctx, &ctx->amg_zt64, (size_t)n))) return r;
+    ctx->amg_T = true;
     k_to_f32_pair<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, ctx->d_pair[1], ctx->d_EV32);
     amg_refresh(ctx);
     LAUNCHCHK(ctx);
@@ -4194,10 +4264,13 @@ static int adj_solve(ufe_ctx *ctx, double tol, int m, int ks, double omega, int 
     k_normalize<double><<<nb, BLOCK, 0, ctx->stream>>>(n, rr, ctx->adj_nrm + 1, V, ctx->adj_nrm + 4);
     for (int j = 0; j < m; j++) {
       double2 *vj = V + (int64_t)j * n, *zj = Z + (int64_t)j * n;
-      if (mg) amg_apply_T(ctx, mT, omega, vj, zj);
-      else precond_T(ctx, mT, omega, ks, vj, zj);
+      if (mg) {
+        amg_apply_T(ctx, mT, omega, vj, zj, w);
+      } else {
+        precond_T(ctx, mT, omega, ks, vj, zj);
+        apply_AT(ctx, mT, ar, zj, w);
+      }
       used += mg ? 2 * ks : ks;
-      apply_AT(ctx, mT, ar, zj, w);
       (*matvecs)++;
       double *h1 = ctx->adj_H1 + (int64_t)j * 65;
       k_multi_dot<double><<<DOT_BLOCKS, BLOCK, 0, ctx->stream>>>(n, j + 1, ar, V, w, ctx->kry_part);
