@@ -138,3 +138,35 @@ def test_sor_loop_on_patches_stops_as_the_sweeps_do():
     wl = geometry.marine(12000, seed=5, picard=2)
     wl.params.use_analytical_GL_flux = True
     _same_step(wl)
+
+
+# one patch width below 131,072 points and the other above, one sweep and two
+@pytest.mark.parametrize("n,nu,gl", [(300, 2, False), (6000, 1, False), (6000, 2, True), (36000, 2, False)])
+def test_transposed_smoothing_on_patches_is_bit_identical(n, nu, gl):
+    """The adjoint's preconditioner and operator on patches against the colour passes."""
+    torch = pytest.importorskip("torch")
+    from ufemism_amd.adjoint import AdjointOptions, SSAProblem, ssa_velocities
+    print(f"[patch] adjoint {n} nu {nu} gl {gl}", flush=True)
+    wl = geometry.marine(n, seed=5, picard=2)
+    wl.params.use_analytical_GL_flux = gl
+    out = {}
+    for on in ("0", "1"):
+        os.environ["UFE_AMG_PATCH"] = on
+        ctx = abi.Context(0)
+        try:
+            step = Step(ctx, wl)
+            ctx.update_general_ice_model_data()
+            prob = SSAProblem(ctx, AdjointOptions(picard_iterations=2, lin_rel_tol=1e-10, gmres_restart=20,
+                                                  precond_sweeps=nu, precond_type=abi.UFE_PRECOND_MULTIGRID))
+            tau = torch.tensor(wl.tau_c_override(step.ma["VAaAc"]), dtype=torch.float64, device=prob.dev)
+            lt = torch.log(tau).requires_grad_(True)
+            A = torch.full_like(tau, wl.A_flow).requires_grad_(True)
+            U, V = ssa_velocities(lt, A, prob)
+            (U * U + 2.0 * V * V).sum().backward()
+            out[on] = (prob.backward_stats.adjoint_matvecs, lt.grad.clone(), A.grad.clone(), U.detach().clone())
+        finally:
+            ctx.close()
+            os.environ.pop("UFE_AMG_PATCH", None)
+    assert out["0"][0] == out["1"][0] > 0
+    for a, b in zip(out["0"][1:], out["1"][1:]):
+        assert torch.equal(a, b) and float(a.abs().max()) > 0
