@@ -3720,6 +3720,22 @@ static int64_t precond_passes(const ufe_ctx *ctx, int ks) {
   return 5 * (int64_t)ks - (ctx->repeat_turn ? 0 : (int64_t)(ks - 1));
 }
 
+// h = V^T w for k vectors
+extern "C++" template <typename T>
+static void orth_coeffs(ufe_ctx *ctx, int k, const ActiveRanges &ar, const typename V2T<T>::t *V,
+                        const typename V2T<T>::t *w, double *h) {
+  k_multi_dot<T><<<DOT_BLOCKS, BLOCK, 0, ctx->stream>>>(ctx->nA, k, ar, V, w, ctx->kry_part);
+  k_multi_dot_reduce<<<k, 256, 0, ctx->stream>>>(DOT_BLOCKS, k, ctx->kry_part, h, 0);
+}
+// the last Gram-Schmidt pass: h = V^T w, w -= V h, next = w / |w| and the norm
+extern "C++" template <typename T>
+static void orth_step(ufe_ctx *ctx, int k, const ActiveRanges &ar, const typename V2T<T>::t *V,
+                      typename V2T<T>::t *w, double *h, typename V2T<T>::t *next, double *norm) {
+  orth_coeffs<T>(ctx, k, ar, V, w, h);
+  k_multi_axpy_norm<T><<<DOT_BLOCKS, BLOCK, 0, ctx->stream>>>(ctx->nA, k, ar, V, h, w, ctx->kry_part);
+  k_normalize_parts<T><<<nblk(ctx->nA), BLOCK, 0, ctx->stream>>>(ctx->nA, w, DOT_BLOCKS, ctx->kry_part, next, norm);
+}
+
 // One GMRES(m) cycle on A d = r (r held in R32 or kry_R64 with |r|^2 in d_scalar[1]),
 // then w += d in FP64.  Templated on the Krylov precision.  target > 0: every
 // GMRES_CHECK iterations the least-squares residual is evaluated on the host
@@ -3770,19 +3786,11 @@ static int gmres_cycle(ufe_ctx *ctx, int m, int ksweeps, double omega, int passe
     (*matvecs)++;
     // classical Gram-Schmidt, one or two passes
     double *h1 = ctx->kry_H1 + (int64_t)j * 65, *h2 = ctx->kry_H2 + (int64_t)j * 65;
-    k_multi_dot<T><<<DOT_BLOCKS, BLOCK, 0, ctx->stream>>>(n, j + 1, ar, V, w, ctx->kry_part);
-    k_multi_dot_reduce<<<j + 1, 256, 0, ctx->stream>>>(DOT_BLOCKS, j + 1, ctx->kry_part, h1, 0);
-    k_multi_axpy<T><<<nb, BLOCK, 0, ctx->stream>>>(n, j + 1, V, h1, w);
     if (passes > 1) {
-      k_multi_dot<T><<<DOT_BLOCKS, BLOCK, 0, ctx->stream>>>(n, j + 1, ar, V, w, ctx->kry_part);
-      k_multi_dot_reduce<<<j + 1, 256, 0, ctx->stream>>>(DOT_BLOCKS, j + 1, ctx->kry_part, h2, 0);
-      k_multi_axpy<T><<<nb, BLOCK, 0, ctx->stream>>>(n, j + 1, V, h2, w);
-    } else {
-      k_fill<double><<<1, 64, 0, ctx->stream>>>(h2, j + 1, 0.0);
+      orth_coeffs<T>(ctx, j + 1, ar, V, w, h1);
+      k_multi_axpy<T><<<nb, BLOCK, 0, ctx->stream>>>(n, j + 1, V, h1, w);
     }
-    k_multi_dot<T><<<DOT_BLOCKS, BLOCK, 0, ctx->stream>>>(n, 1, ar, w, w, ctx->kry_part);
-    k_multi_dot_reduce<<<1, 256, 0, ctx->stream>>>(DOT_BLOCKS, 1, ctx->kry_part, ctx->kry_nrm, 0);
-    k_normalize<T><<<nb, BLOCK, 0, ctx->stream>>>(n, w, ctx->kry_nrm, V + (int64_t)(j + 1) * n, ctx->kry_Hs + j);
+    orth_step<T>(ctx, j + 1, ar, V, w, passes > 1 ? h2 : h1, V + (int64_t)(j + 1) * n, ctx->kry_Hs + j);
     if (target > 0.0 && j + 1 < m && (j + 1) % GMRES_CHECK == 0) {
       const int k = j + 1;
       std::vector<double> yy;
@@ -3790,7 +3798,7 @@ static int gmres_cycle(ufe_ctx *ctx, int m, int ksweeps, double omega, int passe
       if (const int e = kry_readback(ctx, &hb)) return e;
       double res = HUGE_VAL;
       const double beta = std::sqrt(hb[KRY_HBLOCK - 4 + 1]);
-      hessenberg_lsq(k, hb, hb + 65 * 64, hb + 2 * 65 * 64, beta, yy, &res);
+      hessenberg_lsq(k, hb, passes > 1 ? hb + 65 * 64 : nullptr, hb + 2 * 65 * 64, beta, yy, &res);
       if (res <= target * beta) {
         m = k;
         break;
@@ -3803,7 +3811,8 @@ static int gmres_cycle(ufe_ctx *ctx, int m, int ksweeps, double omega, int passe
   if (const int e = kry_readback(ctx, &hb)) return e;
   prof_collect(ctx);
   std::vector<double> y;
-  const int kk = hessenberg_lsq(m, hb, hb + 65 * 64, hb + 2 * 65 * 64, std::sqrt(hb[KRY_HBLOCK - 4 + 1]), y);
+  const int kk = hessenberg_lsq(m, hb, passes > 1 ? hb + 65 * 64 : nullptr, hb + 2 * 65 * 64,
+                                std::sqrt(hb[KRY_HBLOCK - 4 + 1]), y);
   if (kk == 0) return UFE_OK;
   double *hy = ctx->h_kry + KRY_HBLOCK;   // pinned: the copy reads it after this call returns
   std::copy(y.begin(), y.begin() + kk, hy);
@@ -4272,14 +4281,7 @@ static int adj_solve(ufe_ctx *ctx, double tol, int m, int ks, double omega, int 
       }
       used += mg ? 2 * ks : ks;
       (*matvecs)++;
-      double *h1 = ctx->adj_H1 + (int64_t)j * 65;
-      k_multi_dot<double><<<DOT_BLOCKS, BLOCK, 0, ctx->stream>>>(n, j + 1, ar, V, w, ctx->kry_part);
-      k_multi_dot_reduce<<<j + 1, 256, 0, ctx->stream>>>(DOT_BLOCKS, j + 1, ctx->kry_part, h1, 0);
-      k_multi_axpy<double><<<nb, BLOCK, 0, ctx->stream>>>(n, j + 1, V, h1, w);
-      k_multi_dot<double><<<DOT_BLOCKS, BLOCK, 0, ctx->stream>>>(n, 1, ar, w, w, ctx->kry_part);
-      k_multi_dot_reduce<<<1, 256, 0, ctx->stream>>>(DOT_BLOCKS, 1, ctx->kry_part, ctx->adj_nrm + 5, 0);
-      k_normalize<double><<<nb, BLOCK, 0, ctx->stream>>>(n, w, ctx->adj_nrm + 5, V + (int64_t)(j + 1) * n,
-                                                        ctx->adj_Hs + j);
+      orth_step<double>(ctx, j + 1, ar, V, w, ctx->adj_H1 + (int64_t)j * 65, V + (int64_t)(j + 1) * n, ctx->adj_Hs + j);
     }
     LAUNCHCHK(ctx);
     HIPCHK(ctx, hipMemcpyAsync(H1.data(), ctx->adj_H1, sizeof(double) * 65 * m, hipMemcpyDeviceToHost, ctx->stream));
