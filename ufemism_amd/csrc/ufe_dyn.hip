@@ -2239,6 +2239,7 @@ constexpr int AMG_COARSE_SWEEPS = 20;    // coarsest level too large for the den
 constexpr size_t AMG_TAIL_LDS_MARGIN = 256;     // bytes of LDS left unused by k_amg_tail
 constexpr int AMG_FUSE_MAX_POINTS = 1 << 24;   // levels up to this size take the fused cycle kernels
 constexpr size_t AMG_FUSE_LDS_MAX = 56 * 1024;  // their LDS arrays (36 bytes per listed point; 6 KiB static beside)
+constexpr size_t AMG_FUSE_LDS_HELD = 58 * 1024; // and with the rows: 64 KiB less the static part
 
 // Coarse levels of at most this many points get the fused kernels' blocks and
 // halos when their block lists fit in LDS (UFE_AMG_FUSE_MAX=n sets the size
@@ -2530,7 +2531,18 @@ static int amg_setup(ufe_ctx *ctx) {
             (r = dupload(ctx, &d_glo, H.glo.data(), H.glo.size())))
           return r;
         V.F = AmgFuse{H.depth, d_ext_ptr, d_ext, d_cnt, d_rstart, d_rptr, d_lcol, d_lcf, V.S, nullptr,
-                      d_gptr, d_gagg, d_glo, H.max_ext};
+                      d_gptr, d_gagg, d_glo, H.max_ext, 0, 0};
+        // the blocks' rows beside the lists where both orientations fit
+        int nnz = 0, rows = 0;
+        for (int b = 0; b < H.nblocks; b++) {
+          const int q0 = H.rstart[b], q1 = H.rstart[b + 1];
+          rows = std::max(rows, q1 - q0);
+          nnz = std::max(nnz, H.rptr[q1] - H.rptr[q0]);
+          if (H.transposed_ok) nnz = std::max(nnz, H.rptrT[q1] - H.rptrT[q0]);
+        }
+        V.F.nnz_cap = nnz;
+        V.F.row_cap = rows;
+        if (amg_fuse_lds(V.F) > AMG_FUSE_LDS_HELD) V.F.nnz_cap = V.F.row_cap = 0;
         V.fuse_blocks = H.nblocks;
         V.blocks = true;
         V.fuse = fuse_on;
@@ -2703,7 +2715,8 @@ static void amg_cycle(ufe_ctx *ctx, int l, const float2 *b, float2 *x, AmgDots *
   const int nu = std::max(1, ctx->amg_nu);
   if (amg_fused_cycle(ctx, l)) {   // two kernels with block halos, same results
     AmgLevel &C = ctx->amg[l + 1];
-    const size_t lds = (size_t)V.F.cap * 36;
+    const size_t lds = amg_fuse_lds(V.F);
+    const bool held = V.F.nnz_cap > 0;
     AmgFuse F = V.F;
     if (ctx->amg_T) {
       F.rptr = V.fuse_rptrT;
@@ -2712,7 +2725,8 @@ static void amg_cycle(ufe_ctx *ctx, int l, const float2 *b, float2 *x, AmgDots *
     }
     // the blocks are whole aggregates of level l + 1: the pre-smoothing kernel
     // also sums their members' residuals into C.b (as k_amg_gather)
-    k_amg_fuse_pre<<<V.fuse_blocks, AMG_FUSE_BLOCK, lds, ctx->stream>>>(
+    auto pre = held ? k_amg_fuse_pre<true> : k_amg_fuse_pre<false>;
+    pre<<<V.fuse_blocks, AMG_FUSE_BLOCK, lds, ctx->stream>>>(
         F, nu, b, V.t, C.b, AMG_BJ_OMEGA, fold ? fold->w1 : nullptr, fold ? fold->knb : 0,
         fold ? fold->kpart : nullptr, fold ? fold->sc : nullptr, fold ? fold->rc2 : nullptr);
     if (fold) b = fold->rc2;
@@ -2720,7 +2734,8 @@ static void amg_cycle(ufe_ctx *ctx, int l, const float2 *b, float2 *x, AmgDots *
     // a K-step level below leaves its step-2 partials to this kernel (amg_solve_level)
     const int cnd = amg_dot_count(C);
     const bool dot = dots && V.F.depth >= nu + 1;
-    k_amg_fuse_post<<<V.fuse_blocks, AMG_FUSE_BLOCK, lds, ctx->stream>>>(
+    auto post = held ? k_amg_fuse_post<true> : k_amg_fuse_post<false>;
+    post<<<V.fuse_blocks, AMG_FUSE_BLOCK, lds, ctx->stream>>>(
         F, nu, b, V.t, C.agg, C.e1, C.e2, C.kstep ? C.sc : nullptr, C.kstep ? C.part : nullptr, cnd, x,
         AMG_BJ_OMEGA, dot ? dots->a : nullptr, dot && dots->c_rhs ? 1 : 0, dot ? dots->y : nullptr,
         dot ? dots->part : nullptr);
