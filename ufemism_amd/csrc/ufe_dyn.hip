@@ -2664,6 +2664,23 @@ static bool amg_fused_cycle(const ufe_ctx *ctx, int l) {
   return l >= 1 && V.fuse && (!ctx->amg_T || V.fuseT) && std::max(1, ctx->amg_nu) <= V.F.depth;
 }
 
+// K-step partial sums of level V: one per fused-kernel block when it has them
+static int amg_dot_count(const AmgLevel &V) {
+  return V.blocks ? V.fuse_blocks : std::min(AMG_DOT_BLOCKS, nblk(V.n, 256));
+}
+
+// Level 1's step-2 coefficients: added up by every block of the fine prolongation
+// up to AMG_LATE_KFIN blocks of it, by a launch of their own (4 us) above, where the
+// blocks' reading of the partial sums (6 KB each) takes longer than that
+constexpr int AMG_LATE_KFIN = 1024;
+static bool amg_late_kfin(const ufe_ctx *ctx) { return nblk(ctx->nA) <= AMG_LATE_KFIN; }
+static AmgStep2 amg_fine_step2(const ufe_ctx *ctx) {
+  const AmgLevel &C = ctx->amg[1];
+  if (!C.kstep) return {nullptr, nullptr, 0};
+  if (!amg_late_kfin(ctx)) return {C.sc, nullptr, 0};
+  return {C.sc, C.part, amg_dot_count(C)};
+}
+
 // The K-step dots of a cycle's result (y = A x, and y.a, y.y, y.c by block),
 // which the fused post-smoothing computes itself when its halos reach one ring
 // beyond the smoothing; done reports whether it did.
@@ -2674,11 +2691,6 @@ struct AmgDots {
   double *part;
   bool done;
 };
-
-// K-step partial sums of level V: one per fused-kernel block when it has them
-static int amg_dot_count(const AmgLevel &V) {
-  return V.blocks ? V.fuse_blocks : std::min(AMG_DOT_BLOCKS, nblk(V.n, 256));
-}
 
 // The step-1 finish of a K-step (alpha1 from the partials, rc2 = b - alpha1 w1)
 // done by the second cycle's fused pre-smoothing kernel (amg_kfold_max).
@@ -2752,7 +2764,8 @@ static void amg_cycle(ufe_ctx *ctx, int l, const float2 *b, float2 *x, AmgDots *
   k_amg_residual<<<nb, BLOCK, 0, ctx->stream>>>(A, cur, b, V.r);
   k_amg_gather<<<nblk(C.n), BLOCK, 0, ctx->stream>>>(C.n, C.mptr, C.mem, V.r, nullptr, C.b);
   amg_solve_level(ctx, l + 1);
-  k_amg_prolong<<<nb, BLOCK, 0, ctx->stream>>>(V.n, C.agg, C.e1, C.e2, C.kstep ? C.sc : nullptr, cur, nullptr);
+  k_amg_prolong<<<nb, BLOCK, 0, ctx->stream>>>(V.n, C.agg, C.e1, C.e2, AmgStep2{C.kstep ? C.sc : nullptr, nullptr, 0},
+                                               cur, nullptr);
   for (int s = 0; s < nu; s++) {
     k_amg_bj<<<nb, BLOCK, 0, ctx->stream>>>(A, b, cur, oth, AMG_BJ_OMEGA);
     std::swap(cur, oth);
@@ -2847,7 +2860,7 @@ static void amg_solve_level(ufe_ctx *ctx, int l) {
   }
   // the step-2 coefficients: computed by the fused post-smoothing of the level
   // above from these partials, or here for the other prolongations
-  if (!amg_fused_cycle(ctx, l - 1)) k_amg_kfin<<<1, 256, 0, ctx->stream>>>(nd, V.part, V.sc, 2);
+  if (!amg_fused_cycle(ctx, l - 1) && !(l == 1 && amg_late_kfin(ctx))) k_amg_kfin<<<1, 256, 0, ctx->stream>>>(nd, V.part, V.sc, 2);
 }
 
 // The coarse levels of one application (level 1's b in, e1, e2 and sc out)
@@ -3135,13 +3148,13 @@ static bool amg_apply(ufe_ctx *ctx, const AaAcMesh &am, float omega, const float
   if (!launched) amg_solve_level(ctx, 1);
   const uint8_t *skip = ctx->gl_active ? ctx->d_skip : nullptr;
   if (patches) {
-    k_amg_prolong_neumann<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, C.agg, C.e1, C.e2, C.kstep ? C.sc : nullptr,
+    k_amg_prolong_neumann<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, C.agg, C.e1, C.e2, amg_fine_step2(ctx),
                                                              ctx->amg_zt, skip, ctx->amg_zu, neu_list(ctx),
                                                              cor_list(ctx), ctx->d_place);
     patch_smooth(ctx, true, omega, v, ctx->amg_zu, z, w);
     return w != nullptr;
   }
-  k_amg_prolong<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, C.agg, C.e1, C.e2, C.kstep ? C.sc : nullptr, z, skip);
+  k_amg_prolong<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, C.agg, C.e1, C.e2, amg_fine_step2(ctx), z, skip);
   neumann_f32(ctx, z);
   for (int k = 0; k < nu; k++) enqueue_sweep_fp32(ctx, am, omega, z, v, true, false, k == nu - 1);
   return false;
@@ -3241,7 +3254,7 @@ static void amg_apply_T(ufe_ctx *ctx, const AaAcMesh &mT, double omega, const do
     if (!launched) (void)hipGetLastError();
   }
   if (!launched) amg_solve_level(ctx, 1);   // the same kernels, eager
-  k_amg_prolong64<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, C.agg, C.e1, C.e2, C.kstep ? C.sc : nullptr, zt, skip);
+  k_amg_prolong64<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, C.agg, C.e1, C.e2, amg_fine_step2(ctx), zt, skip);
   if (patches) {
     patch_smooth_T(ctx, mT, true, omega, v, zt, z, w);
     return;
