@@ -4987,9 +4987,7 @@ int ufe_op_derivatives_AaAc(ufe_ctx *ctx, const double *d, double *ddx, double *
   NEED_MESH(ctx);
   const int n = ctx->nA;
   k_gather_perm<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, ctx->d_perm, d, ctx->d_tmp[0]);
-  k_deriv_AaAc<<<nblk(n), BLOCK, 0, ctx->stream>>>(aaac_mesh(ctx), ctx->d_tmp[0], ctx->d_tmp[1], ctx->d_tmp[2]);
-  k_scatter_perm<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, ctx->d_perm, ctx->d_tmp[1], ddx);
-  k_scatter_perm<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, ctx->d_perm, ctx->d_tmp[2], ddy);
+  k_deriv_AaAc<<<xcd_grid(n), BLOCK, 0, ctx->stream>>>(aaac_mesh(ctx), ctx->d_perm, ctx->d_tmp[0], ddx, ddy);
   LAUNCHCHK(ctx);
   return ufe_synchronize(ctx);
 }
@@ -4997,20 +4995,15 @@ int ufe_op_curvatures_AaAc(ufe_ctx *ctx, const double *d, double *a, double *b, 
   NEED_MESH(ctx);
   const int n = ctx->nA;
   k_gather_perm<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, ctx->d_perm, d, ctx->d_tmp[0]);
-  k_curv_AaAc<<<nblk(n), BLOCK, 0, ctx->stream>>>(aaac_mesh(ctx), ctx->d_tmp[0], ctx->d_tmp[1], ctx->d_tmp[2], ctx->d_tmp[3]);
-  k_scatter_perm<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, ctx->d_perm, ctx->d_tmp[1], a);
-  k_scatter_perm<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, ctx->d_perm, ctx->d_tmp[2], b);
-  k_scatter_perm<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, ctx->d_perm, ctx->d_tmp[3], c);
+  k_curv_AaAc<<<nblk(n), BLOCK, 0, ctx->stream>>>(aaac_mesh(ctx), ctx->d_perm, ctx->d_tmp[0], a, b, c);
   LAUNCHCHK(ctx);
   return ufe_synchronize(ctx);
 }
 int ufe_op_neumann_AaAc(ufe_ctx *ctx, double *d) {
   NEED_MESH(ctx);
-  const int n = ctx->nA;
-  k_gather_perm<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, ctx->d_perm, d, ctx->d_tmp[0]);
-  if (ctx->n_neu) k_neumann_scalar<<<nblk(ctx->n_neu), BLOCK, 0, ctx->stream>>>(neu_list(ctx), ctx->d_tmp[0]);
-  k_neumann_scalar_serial<<<1, 64, 0, ctx->stream>>>(cor_list(ctx), ctx->d_tmp[0]);
-  k_scatter_perm<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, ctx->d_perm, ctx->d_tmp[0], d);
+  if (ctx->n_neu)
+    k_neumann_scalar<<<nblk(ctx->n_neu), BLOCK, 0, ctx->stream>>>(neu_list(ctx), ctx->d_perm, d);
+  k_neumann_scalar<<<nblk(ctx->n_cor, 64), 64, 0, ctx->stream>>>(cor_list(ctx), ctx->d_perm, d);
   LAUNCHCHK(ctx);
   return ufe_synchronize(ctx);
 }
