@@ -42,6 +42,15 @@ inline void amg_parts(int n, int parts, F body) {
   for (auto &x : th) x.join();
 }
 
+// The coupling that place i of a block reads ahead of its use: the block's nn
+// couplings start at k0 of the level's array (which is not empty), places past
+// their end read the last one again.  A block without couplings reads the one
+// before its start, never the one after: k0 may be the array's length.
+constexpr int amg_held_index(int k0, int nn, int i) {
+  const int k = k0 + (i < nn - 1 ? i : nn - 1);
+  return k > 0 ? k : 0;
+}
+
 // Rows built in parts: part t holds the rows of its range one after another,
 // rowlen[i] the length of row i.  Joins them into CSR ptr, col, cf.
 template <typename T>

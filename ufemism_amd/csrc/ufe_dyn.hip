@@ -22,9 +22,9 @@
 #include <hip/hip_ext.h>
 #include <type_traits>
 
-#include "ufe_kernels.inc"
 #include "amg_host.h"
 #include "patch_host.h"
+#include "ufe_kernels.inc"
 #include "patch_kernels.inc"
 
 namespace ufe {
