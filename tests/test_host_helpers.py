@@ -48,3 +48,35 @@ int main() {
   return 0;
 }
 """)
+
+
+def test_patch_buffers_are_made_each_on_its_own(run_driver):
+    """A call that fails or finds no room at any of the buffers leaves the others
+    to the next call, which makes what is missing and nothing twice."""
+    run_driver("spaces", r"""
+#include <cstdio>
+#include "patch_host.h"
+int main() {
+  for (int stop = 0; stop < 3; stop++)          // the buffer that is refused
+    for (int code : {0, 7}) {                   // no room, or an error
+      int made = 0, x[3];
+      int *a = nullptr, *b = nullptr, *c = nullptr;
+      auto make = [&](int *&p) {
+        if (made == stop) return code;
+        p = &x[made++];
+        return 0;
+      };
+      const int r = ufe::patch_spaces(make, a, b, c);
+      if (r != code || (a && b && c)) return std::printf("refused at %d: status %d\n", stop, r), 1;
+      int made2 = made;
+      auto make2 = [&](int *&p) {
+        p = &x[made2++];
+        return 0;
+      };
+      const int r2 = ufe::patch_spaces(make2, a, b, c);
+      if (r2 || !a || !b || !c || made2 != 3 || a == b || b == c || a == c)
+        return std::printf("after a refusal at %d: status %d, %d made\n", stop, r2, made2), 1;
+    }
+  return 0;
+}
+""")

@@ -59,6 +59,17 @@ struct PatchHost {                // a part of the patches, one after another
 
 constexpr int PATCH_BASE_BITS = 27;
 
+// The buffers beside the patches: makes those that are not there yet, each on its
+// own, so that a call after one that stopped half-way makes the rest.  make(p)
+// returns 0, with p still null where there is no room, or an error, which ends
+// this; the patches may be used only once every buffer is there.
+template <typename Make, typename... P>
+inline int patch_spaces(Make make, P *&...p) {
+  int r = 0;
+  ((r = r || p ? r : make(p)), ...);
+  return r;
+}
+
 // All points along the Hilbert order (member by member): the rows of a colour
 // are sorted already, so this is a merge of the five colours and the rest, in
 // as many key ranges as there are host threads.

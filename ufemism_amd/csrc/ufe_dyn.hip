@@ -198,6 +198,7 @@ struct ufe_ctx {
   double2 *sor_w1 = nullptr;        // second buffer of the SOR loop on patches
   uint32_t *sor_reports = nullptr;
   uint32_t sor_epoch = 0;           // sweeps reported in sor_reports so far
+  bool sor_ready = false;           // the loop's buffers are there and sor_reports is cleared
   int32_t *d_place = nullptr;       // 0: SOR row; k: edge point k - 1; -k: corner k - 1
   uint8_t *d_skip = nullptr;        // SOR rows prescribed by the grounding-line flux
   bool gl_active = false;
@@ -448,6 +449,7 @@ static void free_mesh(ufe_ctx *ctx) {
   ctx->d_place = nullptr;
   ctx->sor_w1 = nullptr;
   ctx->sor_reports = nullptr;
+  ctx->sor_ready = false;
   ctx->h_key.clear();
   ctx->h_mid.clear();
   ctx->amg_zt = ctx->amg_zu = nullptr;
@@ -2932,7 +2934,23 @@ static PatchShape patch_shape(const ufe_ctx *ctx, PatchKind k) {
   return {std::max(64, std::min(240, ctx->nA / 256)), 256};
 }
 
-// The parts of one patch set in one device allocation
+// Device memory for the patches.  They are one of two ways to the same results, so
+// where there is no room p stays null and the colour launches run instead.
+extern "C++" template <typename T>
+static int patch_alloc(ufe_ctx *ctx, T *&p, size_t n) {
+  void *q = nullptr;
+  const hipError_t e = hipMalloc(&q, std::max(n, (size_t)1) * sizeof(T));
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    return UFE_OK;
+  }
+  HIPCHK(ctx, e);
+  ctx->allocs.push_back(q);
+  p = static_cast<T *>(q);
+  return UFE_OK;
+}
+
+// The parts of one patch set in one device allocation (S.P.d null: no room)
 static int patch_upload(ufe_ctx *ctx, const std::vector<PatchHost> &parts, PatchSet &S) {
   char *base = nullptr;
   size_t total = 0;
@@ -2963,7 +2981,8 @@ static int patch_upload(ufe_ctx *ctx, const std::vector<PatchHost> &parts, Patch
         (r = put(&PatchHost::ncol, S.P.ncol)))
       return r;
     if (round == 0) {
-      if ((r = dalloc(ctx, &base, total))) return r;
+      if ((r = patch_alloc(ctx, base, total))) return r;
+      if (!base) return UFE_OK;
       total = 0;
     }
   }
@@ -3008,8 +3027,10 @@ static int patch_prepare(ufe_ctx *ctx, std::initializer_list<PatchKind> kinds, i
     met.insert(met.end(), kc.begin(), kc.begin() + kp[ctx->n_cor]);
     std::sort(met.begin(), met.end());
     ctx->cor_apart = std::adjacent_find(met.begin(), met.end()) == met.end();
-    if ((r = dupload(ctx, &ctx->d_place, place.data(), nA))) return r;
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    int32_t *d_place = nullptr;
+    if ((r = patch_alloc(ctx, d_place, (size_t)nA))) return r;
+    if (d_place) HIPCHK(ctx, hipMemcpy(d_place, place.data(), sizeof(int32_t) * nA, hipMemcpyHostToDevice));
+    ctx->d_place = d_place;
   }
   for (PatchKind k : kinds) {
     PatchSet &S = ctx->patch[k][nu - 1];
@@ -3044,7 +3065,7 @@ static int patch_prepare(ufe_ctx *ctx, std::initializer_list<PatchKind> kinds, i
       if (sor) patch_mark_shared(nA, parts);
       if ((r = patch_upload(ctx, parts, S))) return r;
       S.bs = sh.bs;
-      S.ok = !sor || sor_patch_resident(ctx, S);
+      S.ok = S.P.d && (!sor || sor_patch_resident(ctx, S));
     }
     S.built = true;
   }
@@ -3064,15 +3085,12 @@ static int amg_patches(ufe_ctx *ctx) {
   }
   int r;
   if ((r = patch_prepare(ctx, {PATCH_PRE32, PATCH_POST32}, nu))) return r;
-  if (!ctx->amg_zt) {
-    if ((r = dalloc(ctx, &ctx->amg_zt, (size_t)ctx->nA))) return r;
-    if ((r = dalloc(ctx, &ctx->amg_zu, (size_t)ctx->nA))) return r;
-  }
-  return UFE_OK;
+  return patch_spaces([&](auto *&p) { return patch_alloc(ctx, p, (size_t)ctx->nA); }, ctx->amg_zt, ctx->amg_zu);
 }
 static bool amg_on_patches(const ufe_ctx *ctx) {
   const int nu = std::max(1, ctx->amg_nu);
-  return nu <= 2 && ctx->patch[PATCH_PRE32][nu - 1].ok && ctx->patch[PATCH_POST32][nu - 1].ok;
+  return nu <= 2 && ctx->patch[PATCH_PRE32][nu - 1].ok && ctx->patch[PATCH_POST32][nu - 1].ok && ctx->d_place &&
+         ctx->amg_zt && ctx->amg_zu;
 }
 
 // One smoothing on patches: from zero with the fine residual into y (pre), or
@@ -3313,6 +3331,20 @@ static int sor_batch(ufe_ctx *ctx, const AaAcMesh &m, double omega, double tol, 
   return UFE_OK;
 }
 
+// The buffers of the sweep loop on patches; sor_ready stays false where there is no room
+static int sor_spaces(ufe_ctx *ctx) {
+  auto vectors = [&](auto *&p) { return patch_alloc(ctx, p, (size_t)ctx->nA); };
+  auto words = [&](auto *&p) { return patch_alloc(ctx, p, (size_t)SOR_REPORT_WORDS); };
+  int r;
+  if ((r = patch_spaces(vectors, ctx->sor_w1)) || (r = patch_spaces(words, ctx->sor_reports))) return r;
+  if (!ctx->sor_w1 || !ctx->sor_reports) return UFE_OK;
+  k_fill<uint32_t><<<nblk(SOR_REPORT_WORDS), BLOCK, 0, ctx->stream>>>(ctx->sor_reports, SOR_REPORT_WORDS, 0u);
+  LAUNCHCHK(ctx);
+  ctx->sor_epoch = 0;
+  ctx->sor_ready = true;
+  return UFE_OK;
+}
+
 // The sweep loop on patches (k_patch_sor): one launch per solve instead of seven
 // per sweep, the same sweeps and bits.  Not used while kernel times are sampled
 // (the sample is per colour launch), on meshes whose patches exceed a workgroup
@@ -3329,12 +3361,10 @@ static const PatchSet *sor_patches(ufe_ctx *ctx, int *err) {
       return nullptr;
     }
     if ((*err = patch_prepare(ctx, {PATCH_SOR64}, 1))) return nullptr;
-    if (S.ok) {
-      if ((*err = dalloc(ctx, &ctx->sor_w1, (size_t)ctx->nA))) return nullptr;
-      if ((*err = dalloc(ctx, &ctx->sor_reports, (size_t)SOR_REPORT_WORDS))) return nullptr;
-      k_fill<uint32_t><<<nblk(SOR_REPORT_WORDS), BLOCK, 0, ctx->stream>>>(ctx->sor_reports, SOR_REPORT_WORDS, 0u);
-      ctx->sor_epoch = 0;
-    }
+  }
+  if (S.ok && !ctx->sor_ready) {
+    if ((*err = sor_spaces(ctx))) return nullptr;
+    if (!ctx->sor_ready) S.ok = false;
   }
   return S.ok ? &S : nullptr;
 }
@@ -4265,7 +4295,7 @@ static int adj_solve(ufe_ctx *ctx, double tol, int m, int ks, double omega, int 
     if ((r = amg_setup(ctx))) return r;
     ctx->amg_nu = ks;
     if ((r = amg_patches(ctx))) return r;
-    if (amg_on_patches(ctx) && !ctx->amg_zt64 && (r = dalloc(ctx, &ctx->amg_zt64, (size_t)n))) return r;
+    if (amg_on_patches(ctx) && !ctx->amg_zt64 && (r = patch_alloc(ctx, ctx->amg_zt64, (size_t)n))) return r;
     ctx->amg_T = true;
     k_to_f32_pair<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, ctx->d_pair[1], ctx->d_EV32);
     amg_refresh(ctx);
