@@ -361,6 +361,20 @@ typedef struct ufe_multigrid_info {
   int32_t fuse_list_max[16];        /* its longest block list (own points and halo) */
 } ufe_multigrid_info;
 int ufe_multigrid_info_get(ufe_ctx *ctx, ufe_multigrid_info *out);
+
+/* Which of two ways to the same results ran in this context so far, counted when
+ * the host queues the work (in a captured graph once).  No counterpart in the
+ * reference. */
+typedef struct ufe_path_counts {
+  int64_t sor_patch;                /* launches of the reference SOR loop on patches */
+  int64_t sor_gave_up;              /* those whose workgroups stopped waiting for each other; the
+                                       colour launches repeat their sweeps */
+  int64_t sor_colour;               /* batches of its sweeps by colour launches */
+  int64_t smooth_patch, smooth_colour;       /* multigrid applications with the fine smoothing on
+                                                patches, by colour launches */
+  int64_t smooth_T_patch, smooth_T_colour;   /* the transposed ones of the adjoint */
+} ufe_path_counts;
+int ufe_path_counts_get(ufe_ctx *ctx, ufe_path_counts *out);
 /* FP64 relative residual of the current velocities. */
 int ufe_ssa_residual(ufe_ctx *ctx, double *rel_residual);
 

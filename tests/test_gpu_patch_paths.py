@@ -1,0 +1,55 @@
+"""Which of two ways to the same results ran: the loop and the smoothing on
+patches, or the colour launches that they replace."""
+import os
+
+import numpy as np
+import pytest
+
+from ufemism_amd import abi, geometry
+from ufemism_amd.dynamics import Step
+
+pytestmark = pytest.mark.gpu
+FIELDS = ("U_SSA", "V_SSA", "Ux_SSA_Ac", "Uy_SSA_Ac", "Hi")
+
+
+def _sor_step(wl, sweep_batch=0, **env):
+    """One step; its results and the ways it took.  Environment switches are read per solve or per mesh."""
+    os.environ.update(env)
+    ctx = abi.Context(0)
+    try:
+        out = Step(ctx, wl, sweep_batch=sweep_batch).run()
+        return out, ctx.path_counts()
+    finally:
+        ctx.close()
+        for k in env:
+            os.environ.pop(k, None)
+
+
+def _same(a, b):
+    assert a["sweeps"] == b["sweeps"], (a["sweeps"], b["sweeps"])
+    for k in ("status", "resets", "last_max_residual", "last_RN"):
+        assert getattr(a["stats"], k) == getattr(b["stats"], k), k
+    for k in FIELDS:
+        assert np.array_equal(a[k], b[k], equal_nan=True), k
+
+
+@pytest.mark.parametrize("kind,n", [("dome", 300), ("marine", 12000), ("marine", 37000), ("marine", 70000)])
+def test_sor_loop_that_gives_up_is_repeated_by_colour_launches(kind, n):
+    """No polls at all: every workgroup gives up after its first sweep.  A few
+    polls: some may give up after any sweep, and what they had written is undone."""
+    print(f"[sor wait] {kind} {n}", flush=True)
+    wl = (geometry.dome if kind == "dome" else geometry.marine)(n, seed=5, picard=3)
+    wl.params.SSA_max_residual_UV = 1e-2
+    wl.params.SSA_max_inner_loops = 60
+    ref, c = _sor_step(wl, UFE_SOR_PATCH="0")
+    assert c["sor_patch"] == 0 and c["sor_colour"] > 0
+    out, c = _sor_step(wl, UFE_SOR_SPINS="0")
+    assert c["sor_patch"] == c["sor_gave_up"] == 1 and c["sor_colour"] > 0
+    _same(ref, out)
+    for spins in ("1", "2", "4", "8", "30"):
+        out, c = _sor_step(wl, sweep_batch=7, UFE_SOR_SPINS=spins)
+        print(f"  spins {spins}: {c['sor_patch']} launches, {c['sor_gave_up']} gave up", flush=True)
+        _same(ref, out)
+    out, c = _sor_step(wl)
+    assert c["sor_patch"] >= 1 and c["sor_gave_up"] == c["sor_colour"] == 0
+    _same(ref, out)

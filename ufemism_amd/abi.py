@@ -32,7 +32,7 @@ EXPORTS = [
     "ufe_ctx_create", "ufe_ctx_destroy", "ufe_set_params", "ufe_last_error", "ufe_version",
     "ufe_mesh_build", "ufe_mesh_upload", "ufe_mesh_sizes", "ufe_mesh_geometry",
     "ufe_remap_build", "ufe_remap_field", "ufe_remap_ice_model", "ufe_remap_export",
-    "ufe_multigrid_info_get",
+    "ufe_multigrid_info_get", "ufe_path_counts_get",
     "ufe_field_count", "ufe_field_name", "ufe_field_id", "ufe_field_info", "ufe_field_set",
     "ufe_field_get", "ufe_field_set_device", "ufe_field_get_device",
     "ufe_update_general_ice_model_data", "ufe_ice_physical_properties", "ufe_solve_SIA", "ufe_solve_SSA",
@@ -139,6 +139,11 @@ class LinSolveOpts(ct.Structure):
                 ("orth_passes", ct.c_int32), ("method", ct.c_int32),
                 ("precond_full_sweeps", ct.c_int32), ("precond_neumann_every_sweep", ct.c_int32),
                 ("precond_type", ct.c_int32)]
+
+
+class PathCounts(ct.Structure):
+    _fields_ = [(n, ct.c_int64) for n in ("sor_patch", "sor_gave_up", "sor_colour", "smooth_patch", "smooth_colour",
+                                          "smooth_T_patch", "smooth_T_colour")]
 
 
 class MultigridInfo(ct.Structure):
@@ -534,6 +539,12 @@ class Context:
         o = MultigridInfo()
         self._chk(self.lib.ufe_multigrid_info_get(self.h, ct.byref(o)), "multigrid_info")
         return o.as_dict()
+
+    def path_counts(self) -> dict:
+        """How often each of two ways to the same results ran so far."""
+        o = PathCounts()
+        self._chk(self.lib.ufe_path_counts_get(self.h, ct.byref(o)), "path_counts")
+        return {f[0]: getattr(o, f[0]) for f in PathCounts._fields_}
 
     def set_device(self, name, ptr):
         """Copy a device buffer (reference layout) into a field."""

@@ -196,9 +196,11 @@ struct ufe_ctx {
   std::vector<uint16_t> h_mid;      // batch member of each row (empty: single mesh)
   PatchSet patch[PATCH_KINDS][2];   // by kind and sweeps - 1
   double2 *sor_w1 = nullptr;        // second buffer of the SOR loop on patches
+  double2 *sor_start = nullptr;     // and the velocities that its launch began with
   uint32_t *sor_reports = nullptr;
   uint32_t sor_epoch = 0;           // sweeps reported in sor_reports so far
   bool sor_ready = false;           // the loop's buffers are there and sor_reports is cleared
+  ufe_path_counts paths{};
   int32_t *d_place = nullptr;       // 0: SOR row; k: edge point k - 1; -k: corner k - 1
   uint8_t *d_skip = nullptr;        // SOR rows prescribed by the grounding-line flux
   bool gl_active = false;
@@ -447,7 +449,7 @@ static void free_mesh(ufe_ctx *ctx) {
   for (auto &k : ctx->patch)
     for (PatchSet &S : k) S = PatchSet{};
   ctx->d_place = nullptr;
-  ctx->sor_w1 = nullptr;
+  ctx->sor_w1 = ctx->sor_start = nullptr;
   ctx->sor_reports = nullptr;
   ctx->sor_ready = false;
   ctx->h_key.clear();
@@ -3141,6 +3143,7 @@ static bool amg_apply(ufe_ctx *ctx, const AaAcMesh &am, float omega, const float
   const int n = ctx->nA, nu = std::max(1, ctx->amg_nu);
   const bool patches = amg_on_patches(ctx);
   AmgLevel &C = ctx->amg[1];
+  (patches ? ctx->paths.smooth_patch : ctx->paths.smooth_colour)++;
   if (patches) {
     patch_smooth(ctx, false, omega, v, nullptr, ctx->amg_zt, ctx->amg_y);
   } else {
@@ -3258,6 +3261,7 @@ static void amg_apply_T(ufe_ctx *ctx, const AaAcMesh &mT, double omega, const do
     }
   };
   AmgLevel &C = ctx->amg[1];
+  (patches ? ctx->paths.smooth_T_patch : ctx->paths.smooth_T_colour)++;
   if (patches) {
     patch_smooth_T(ctx, mT, false, omega, v, nullptr, zt, ctx->amg_y64);
   } else {
@@ -3336,8 +3340,8 @@ static int sor_spaces(ufe_ctx *ctx) {
   auto vectors = [&](auto *&p) { return patch_alloc(ctx, p, (size_t)ctx->nA); };
   auto words = [&](auto *&p) { return patch_alloc(ctx, p, (size_t)SOR_REPORT_WORDS); };
   int r;
-  if ((r = patch_spaces(vectors, ctx->sor_w1)) || (r = patch_spaces(words, ctx->sor_reports))) return r;
-  if (!ctx->sor_w1 || !ctx->sor_reports) return UFE_OK;
+  if ((r = patch_spaces(vectors, ctx->sor_w1, ctx->sor_start)) || (r = patch_spaces(words, ctx->sor_reports))) return r;
+  if (!ctx->sor_w1 || !ctx->sor_start || !ctx->sor_reports) return UFE_OK;
   k_fill<uint32_t><<<nblk(SOR_REPORT_WORDS), BLOCK, 0, ctx->stream>>>(ctx->sor_reports, SOR_REPORT_WORDS, 0u);
   LAUNCHCHK(ctx);
   ctx->sor_epoch = 0;
@@ -3387,10 +3391,20 @@ static bool sor_patch_resident(ufe_ctx *ctx, const PatchSet &S) {
   return S.P.np <= SOR_PATCHES && (S.P.np + 7) / 8 * 8 <= per * cus;
 }
 
+// Polls after which a workgroup of the loop gives up (about a second; a sweep's
+// exchange takes a few).  UFE_SOR_SPINS=n in the environment sets it.
+constexpr int SOR_SPINS = 1 << 20;
+static int sor_spins() {
+  const char *e = std::getenv("UFE_SOR_SPINS");
+  char *end = nullptr;
+  const long n = e ? std::strtol(e, &end, 10) : 0;
+  return end == e || n < 0 ? SOR_SPINS : (int)std::min(n, 1l << 30);
+}
+
 static int run_sor_reference(ufe_ctx *ctx, double tol, int max_sweeps, SorFlags *out, double *seconds) {
   const AaAcMesh m = aaac_mesh(ctx);
   const double omega = ctx->params.SSA_SOR_omega;
-  k_sor_flags_init<<<1, 1, 0, ctx->stream>>>(ctx->d_flags);
+  k_sor_flags_init<<<1, 1, 0, ctx->stream>>>(ctx->d_flags, 0);
   LAUNCHCHK(ctx);
   int batch = ctx->params.sweep_batch > 0 ? ctx->params.sweep_batch : 1;
   int queued = 0;
@@ -3399,19 +3413,21 @@ static int run_sor_reference(ufe_ctx *ctx, double tol, int max_sweeps, SorFlags 
   if (const PatchSet *S = max_sweeps > 0 ? sor_patches(ctx, &perr) : (perr = UFE_OK, nullptr)) {
     // a launch holds the device for its sweeps, so a long solve takes several
     int limit = ctx->params.sweep_batch > 0 ? ctx->params.sweep_batch : 1024, swept = 0, top = max_sweeps;
+    int spins = sor_spins();
     PatchDev P = S->P;
     const double2 *cU = ctx->d_cU, *EV = ctx->d_pair[1], *RHS = ctx->d_pair[2];
     const double *Sxy = ctx->d_Sxy;
     const uint8_t *skip = ctx->gl_active ? ctx->d_skip : nullptr;
     double om = omega, tl = tol;
     int nA = ctx->nA;
-    double2 *W0 = ctx->d_pair[0], *W1 = ctx->sor_w1;
+    double2 *W0 = ctx->d_pair[0], *W1 = ctx->sor_w1, *start = ctx->sor_start;
     uint32_t *reports = ctx->sor_reports;
     SorFlags *fl = ctx->d_flags;
-    bool refused = false;
+    bool refused = false, gave_up = false;
     while (true) {
       uint32_t epoch = ctx->sor_epoch;
-      void *args[] = {&P, &cU, &Sxy, &EV, &RHS, &skip, &om, &tl, &top, &limit, &nA, &W0, &W1, &reports, &epoch, &fl};
+      void *args[] = {&P, &cU, &Sxy, &EV, &RHS, &skip, &om, &tl, &top, &limit, &spins, &nA, &W0, &W1,
+                      &start, &reports, &epoch, &fl};
       const hipError_t launch = hipLaunchCooperativeKernel(sor_patch_kernel(S->bs), dim3((P.np + 7) / 8 * 8),
                                                            dim3(S->bs), args, (unsigned)S->lds, ctx->stream);
       // the HIP runtime may refuse cooperative launches that the device's
@@ -3425,13 +3441,24 @@ static int run_sor_reference(ufe_ctx *ctx, double tol, int max_sweeps, SorFlags 
         break;
       }
       HIPCHK(ctx, launch);
+      ctx->paths.sor_patch++;
       HIPCHK(ctx, hipMemcpyAsync(ctx->h_flags, ctx->d_flags, sizeof(SorFlags), hipMemcpyDeviceToHost, ctx->stream));
       HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+      gave_up = ctx->h_flags->gave_up != 0;
+      if (gave_up) {                 // from where this launch began, by colour launches; for this mesh from here on
+        ctx->paths.sor_gave_up++;
+        ctx->patch[PATCH_SOR64][0].ok = ctx->sor_ready = false;
+        HIPCHK(ctx, hipMemcpyAsync(W0, start, sizeof(double2) * (size_t)nA, hipMemcpyDeviceToDevice, ctx->stream));
+        k_sor_flags_init<<<1, 1, 0, ctx->stream>>>(ctx->d_flags, swept);
+        LAUNCHCHK(ctx);
+        queued = swept;
+        break;
+      }
       ctx->sor_epoch += (uint32_t)(ctx->h_flags->sweep - swept);
       swept = ctx->h_flags->sweep;
       if (ctx->h_flags->done || swept >= max_sweeps) break;
     }
-    if (!refused) {
+    if (!refused && !gave_up) {
       if (seconds) *seconds += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
       *out = *ctx->h_flags;
       return UFE_OK;
@@ -3443,6 +3470,7 @@ static int run_sor_reference(ufe_ctx *ctx, double tol, int max_sweeps, SorFlags 
     const int nb = std::min(batch, max_sweeps - queued);
     int r;
     if ((r = sor_batch(ctx, m, omega, tol, max_sweeps, nb))) return r;
+    ctx->paths.sor_colour++;
     queued += nb;
     HIPCHK(ctx, hipMemcpyAsync(ctx->h_flags, ctx->d_flags, sizeof(SorFlags), hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
@@ -3967,6 +3995,12 @@ static int bicg_inner(ufe_ctx *ctx, int ks, double omega, double reduce, int max
   k_add_to_w<T><<<nb, BLOCK, 0, ctx->stream>>>(n, x, ctx->d_pair[0]);
   neumann_w(ctx);
   LAUNCHCHK(ctx);
+  return UFE_OK;
+}
+
+int ufe_path_counts_get(ufe_ctx *ctx, ufe_path_counts *out) {
+  if (!ctx || !out) return UFE_BAD_INPUT;
+  *out = ctx->paths;
   return UFE_OK;
 }
 
