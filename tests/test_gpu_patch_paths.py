@@ -53,3 +53,27 @@ def test_sor_loop_that_gives_up_is_repeated_by_colour_launches(kind, n):
     out, c = _sor_step(wl)
     assert c["sor_patch"] >= 1 and c["sor_gave_up"] == c["sor_colour"] == 0
     _same(ref, out)
+
+
+def test_loop_of_a_large_mesh_beside_a_smaller_one_of_its_width():
+    """Two meshes whose workgroups have 1,024 threads and whose patches take more
+    than the default 64 KiB of LDS, the larger one solved before and after the smaller."""
+    print("[sor paths] two meshes", flush=True)
+    wls = [geometry.marine(n, seed=5, picard=2) for n in (130000, 90000)]
+    ctxs = [abi.Context(0) for _ in wls]
+    try:
+        steps = []
+        for c, wl in zip(ctxs, wls):
+            wl.params.SSA_max_inner_loops = 5
+            steps.append(Step(c, wl))
+        first = steps[0].run()
+        steps[1].run()
+        steps[0].reset()
+        again = steps[0].run()
+        _same(first, again)
+        for c in ctxs:
+            p = c.path_counts()
+            assert p["sor_patch"] > 0 and p["sor_colour"] == 0, p
+    finally:
+        for c in ctxs:
+            c.close()

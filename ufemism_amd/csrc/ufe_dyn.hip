@@ -3377,13 +3377,25 @@ static const void *sor_patch_kernel(int bs) {
          : bs == 512 ? reinterpret_cast<const void *>(&k_patch_sor<512, false>)
                      : reinterpret_cast<const void *>(&k_patch_sor<1024, true>);
 }
+// The errors by which the runtime declines a cooperative launch: the device has
+// one cooperative queue, and a process beside one that holds it gets
+// hipErrorIllegalState.  Nothing has run then, and the colour launches do the
+// solve.  Any other error is an error of the call.
+constexpr bool sor_launch_declined(hipError_t e) {
+  return e == hipErrorIllegalState || e == hipErrorNotSupported || e == hipErrorCooperativeLaunchTooLarge;
+}
+static_assert(sor_launch_declined(hipErrorIllegalState) && !sor_launch_declined(hipSuccess) &&
+                  !sor_launch_declined(hipErrorInvalidValue) && !sor_launch_declined(hipErrorOutOfMemory) &&
+                  !sor_launch_declined(hipErrorLaunchFailure) && !sor_launch_declined(hipErrorIllegalAddress),
+              "only what declines the launch itself may lead to the colour launches");
 // Whether the device keeps all workgroups of the loop resident
 static bool sor_patch_resident(ufe_ctx *ctx, const PatchSet &S) {
   int coop = 0, cus = 0, per = 0;
   const void *k = sor_patch_kernel(S.bs);
   if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, ctx->device) != hipSuccess || !coop ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess ||
-      hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S.lds) != hipSuccess ||
+      // the limit belongs to the kernel and not to this mesh: never less than another mesh's patches need
+      hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SOR_LDS_MAX) != hipSuccess ||
       hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k, S.bs, S.lds) != hipSuccess) {
     (void)hipGetLastError();
     return false;
@@ -3430,14 +3442,11 @@ static int run_sor_reference(ufe_ctx *ctx, double tol, int max_sweeps, SorFlags 
                       &start, &reports, &epoch, &fl};
       const hipError_t launch = hipLaunchCooperativeKernel(sor_patch_kernel(S->bs), dim3((P.np + 7) / 8 * 8),
                                                            dim3(S->bs), args, (unsigned)S->lds, ctx->stream);
-      // the HIP runtime may refuse cooperative launches that the device's
-      // attributes offer (seen in a host program without torch, on the runtime
-      // of ROCm 7.2: hipErrorIllegalState); nothing has run, so the colour
-      // launches take over, for this mesh from here on
-      refused = launch != hipSuccess && swept == 0;
-      if (refused) {
+      refused = sor_launch_declined(launch);
+      if (refused) {                 // the colour launches go on, for this mesh from here on
         (void)hipGetLastError();
         ctx->patch[PATCH_SOR64][0].ok = false;
+        queued = swept;
         break;
       }
       HIPCHK(ctx, launch);
