@@ -366,6 +366,7 @@ int ufe_multigrid_info_get(ufe_ctx *ctx, ufe_multigrid_info *out);
  * the host queues the work (in a captured graph once).  No counterpart in the
  * reference. */
 typedef struct ufe_path_counts {
+  int64_t patch_sets;               /* sets of patches built on the host */
   int64_t sor_patch;                /* launches of the reference SOR loop on patches */
   int64_t sor_gave_up;              /* those whose workgroups stopped waiting for each other; the
                                        colour launches repeat their sweeps */

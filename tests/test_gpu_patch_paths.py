@@ -1,6 +1,8 @@
 """Which of two ways to the same results ran: the loop and the smoothing on
 patches, or the colour launches that they replace."""
 import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -46,7 +48,7 @@ def test_sor_loop_that_gives_up_is_repeated_by_colour_launches(kind, n):
     out, c = _sor_step(wl, UFE_SOR_SPINS="0")
     assert c["sor_patch"] == c["sor_gave_up"] == 1 and c["sor_colour"] > 0
     _same(ref, out)
-    for spins in ("1", "2", "4", "8", "30"):
+    for spins in ("1", "2", "4", "8", "12", "16", "30"):
         out, c = _sor_step(wl, sweep_batch=7, UFE_SOR_SPINS=spins)
         print(f"  spins {spins}: {c['sor_patch']} launches, {c['sor_gave_up']} gave up", flush=True)
         _same(ref, out)
@@ -77,3 +79,37 @@ def test_loop_of_a_large_mesh_beside_a_smaller_one_of_its_width():
     finally:
         for c in ctxs:
             c.close()
+
+
+CHILD = r"""
+import sys
+sys.modules["torch"] = None          # the HIP runtime the library is linked with
+sys.path.insert(0, sys.argv[1])
+import numpy as np
+from ufemism_amd import abi, geometry
+from ufemism_amd.dynamics import Step
+for n in (300, 2000):
+    ctx = abi.Context(0)
+    out = Step(ctx, geometry.dome(n, seed=5, picard=3)).run()
+    p = ctx.path_counts()
+    print(p, flush=True)
+    assert p["sor_patch"] + p["sor_colour"] > 0
+    assert (p["sor_patch"] > 0) == (p["patch_sets"] > 0), p      # nothing is built that cannot run
+    ctx.close()
+np.save(sys.argv[2], np.stack([out["U_SSA"], out["V_SSA"]]))
+"""
+
+
+def test_process_beside_one_with_the_cooperative_queue(tmp_path):
+    """The device has one cooperative queue: a process that does not get it takes
+    the colour launches, without building the patches of the loop first."""
+    print("[sor paths] second process", flush=True)
+    wl = geometry.dome(2000, seed=5, picard=3)
+    out, c = _sor_step(wl)
+    assert c["sor_patch"] > 0
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-u", "-c", CHILD, root, str(tmp_path / "uv.npy")], capture_output=True, text=True,
+                       timeout=100)
+    print(r.stdout, r.stderr, flush=True)
+    assert r.returncode == 0
+    assert np.array_equal(np.load(tmp_path / "uv.npy"), np.stack([out["U_SSA"], out["V_SSA"]]))

@@ -142,7 +142,7 @@ class LinSolveOpts(ct.Structure):
 
 
 class PathCounts(ct.Structure):
-    _fields_ = [(n, ct.c_int64) for n in ("sor_patch", "sor_gave_up", "sor_colour", "smooth_patch", "smooth_colour",
+    _fields_ = [(n, ct.c_int64) for n in ("patch_sets", "sor_patch", "sor_gave_up", "sor_colour", "smooth_patch", "smooth_colour",
                                           "smooth_T_patch", "smooth_T_colour")]
 
 

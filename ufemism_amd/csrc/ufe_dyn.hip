@@ -3038,6 +3038,7 @@ static int patch_prepare(ufe_ctx *ctx, std::initializer_list<PatchKind> kinds, i
     PatchSet &S = ctx->patch[k][nu - 1];
     if (S.built) continue;
     PatchShape sh = patch_shape(ctx, k);
+    ctx->paths.patch_sets++;
     std::vector<PatchHost> parts;
     const bool sor = k == PATCH_SOR64;
     bool fits = false;
@@ -3349,29 +3350,6 @@ static int sor_spaces(ufe_ctx *ctx) {
   return UFE_OK;
 }
 
-// The sweep loop on patches (k_patch_sor): one launch per solve instead of seven
-// per sweep, the same sweeps and bits.  Not used while kernel times are sampled
-// (the sample is per colour launch), on meshes whose patches exceed a workgroup
-// (about 230,000 vertices), or with UFE_SOR_PATCH=0 in the environment when the
-// mesh is first swept.  Returns the set, or null.
-static const PatchSet *sor_patches(ufe_ctx *ctx, int *err) {
-  *err = UFE_OK;
-  if (ctx->prof) return nullptr;
-  PatchSet &S = ctx->patch[PATCH_SOR64][0];
-  if (!S.built) {
-    const char *off = std::getenv("UFE_SOR_PATCH");
-    if (off && off[0] == '0') {
-      S.built = true;
-      return nullptr;
-    }
-    if ((*err = patch_prepare(ctx, {PATCH_SOR64}, 1))) return nullptr;
-  }
-  if (S.ok && !ctx->sor_ready) {
-    if ((*err = sor_spaces(ctx))) return nullptr;
-    if (!ctx->sor_ready) S.ok = false;
-  }
-  return S.ok ? &S : nullptr;
-}
 static const void *sor_patch_kernel(int bs) {
   return bs == 256 ? reinterpret_cast<const void *>(&k_patch_sor<256, false>)
          : bs == 512 ? reinterpret_cast<const void *>(&k_patch_sor<512, false>)
@@ -3388,12 +3366,77 @@ static_assert(sor_launch_declined(hipErrorIllegalState) && !sor_launch_declined(
                   !sor_launch_declined(hipErrorInvalidValue) && !sor_launch_declined(hipErrorOutOfMemory) &&
                   !sor_launch_declined(hipErrorLaunchFailure) && !sor_launch_declined(hipErrorIllegalAddress),
               "only what declines the launch itself may lead to the colour launches");
+// Whether this process gets cooperative launches on the device, asked before any
+// patch of the loop is built: where it does not, the building and the device
+// memory would be for nothing.  Asked with a launch that has no patch, once per
+// process and device, since the queue that decides it is the process's (a declined
+// request takes 40 ms, the first accepted one 4).
+static int sor_launch_offered(ufe_ctx *ctx, bool *yes) {
+  static std::mutex lock;
+  static std::map<int, bool> offered;
+  const std::lock_guard<std::mutex> guard(lock);
+  const auto known = offered.find(ctx->device);
+  if (known != offered.end()) {
+    *yes = known->second;
+    return UFE_OK;
+  }
+  int coop = 0;
+  HIPCHK(ctx, hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, ctx->device));
+  hipError_t e = hipErrorNotSupported;
+  if (coop) {
+    PatchDev P{};
+    const double2 *cU = nullptr;
+    const double *Sxy = nullptr;
+    const uint8_t *skip = nullptr;
+    double x = 1.0;
+    int n = 0;
+    double2 *W = nullptr;
+    uint32_t *reports = nullptr, epoch = 0;
+    SorFlags *fl = nullptr;
+    void *args[] = {&P, &cU, &Sxy, &cU, &cU, &skip, &x, &x, &n, &n, &n, &n, &W, &W, &W, &reports, &epoch, &fl};
+    e = hipLaunchCooperativeKernel(sor_patch_kernel(256), dim3(8), dim3(256), args, 0, ctx->stream);
+    if (sor_launch_declined(e)) (void)hipGetLastError();
+    else HIPCHK(ctx, e);
+  }
+  offered[ctx->device] = *yes = e == hipSuccess;
+  return UFE_OK;
+}
+
+// The sweep loop on patches (k_patch_sor): one launch per solve instead of seven
+// per sweep, the same sweeps and bits.  Not used while kernel times are sampled
+// (the sample is per colour launch), on meshes whose patches exceed a workgroup
+// (about 230,000 vertices), where cooperative launches are declined, or with
+// UFE_SOR_PATCH=0 in the environment when the mesh is first swept.  Returns the
+// set, or null.
+static const PatchSet *sor_patches(ufe_ctx *ctx, int *err) {
+  *err = UFE_OK;
+  if (ctx->prof) return nullptr;
+  PatchSet &S = ctx->patch[PATCH_SOR64][0];
+  if (!S.built) {
+    const char *off = std::getenv("UFE_SOR_PATCH");
+    if (off && off[0] == '0') {
+      S.built = true;
+      return nullptr;
+    }
+    bool offered = false;
+    if ((*err = sor_launch_offered(ctx, &offered))) return nullptr;
+    if (!offered) {
+      S.built = true;
+      return nullptr;
+    }
+    if ((*err = patch_prepare(ctx, {PATCH_SOR64}, 1))) return nullptr;
+  }
+  if (S.ok && !ctx->sor_ready) {
+    if ((*err = sor_spaces(ctx))) return nullptr;
+    if (!ctx->sor_ready) S.ok = false;
+  }
+  return S.ok ? &S : nullptr;
+}
 // Whether the device keeps all workgroups of the loop resident
 static bool sor_patch_resident(ufe_ctx *ctx, const PatchSet &S) {
-  int coop = 0, cus = 0, per = 0;
+  int cus = 0, per = 0;
   const void *k = sor_patch_kernel(S.bs);
-  if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, ctx->device) != hipSuccess || !coop ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess ||
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess ||
       // the limit belongs to the kernel and not to this mesh: never less than another mesh's patches need
       hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SOR_LDS_MAX) != hipSuccess ||
       hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k, S.bs, S.lds) != hipSuccess) {
