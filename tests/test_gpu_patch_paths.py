@@ -113,3 +113,11 @@ def test_process_beside_one_with_the_cooperative_queue(tmp_path):
     print(r.stdout, r.stderr, flush=True)
     assert r.returncode == 0
     assert np.array_equal(np.load(tmp_path / "uv.npy"), np.stack([out["U_SSA"], out["V_SSA"]]))
+
+
+def test_mesh_too_large_for_the_loop_is_not_walked():
+    print("[sor paths] too large", flush=True)
+    wl = geometry.marine(300000, seed=5, picard=1)
+    wl.params.SSA_max_inner_loops = 2
+    _, c = _sor_step(wl)
+    assert c["patch_sets"] == c["sor_patch"] == 0 and c["sor_colour"] > 0, c

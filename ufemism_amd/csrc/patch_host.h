@@ -70,6 +70,14 @@ inline int patch_spaces(Make make, P *&...p) {
   return r;
 }
 
+// The least that the largest colour of a patch can hold when np patches share the
+// points: a mesh for which this exceeds the workgroup needs no walk to be refused.
+inline int patch_least_group(const int *colour_active, int np) {
+  int most = 0;
+  for (int c = 0; c < 5; c++) most = std::max(most, colour_active[c]);
+  return (most + np - 1) / np;
+}
+
 // All points along the Hilbert order (member by member): the rows of a colour
 // are sorted already, so this is a merge of the five colours and the rest, in
 // as many key ranges as there are host threads.
@@ -127,9 +135,9 @@ inline std::vector<int32_t> patch_order(const PatchMesh &m) {
 // rows).  Built in contiguous parts on the host's threads; the offsets in the
 // descriptors count from the start of the first part, so that the parts are
 // simply put one after another.  Returns false when the mesh does not fit the
-// packed indices.
+// packed indices, or at the first patch with more than group_max rows of a colour.
 inline bool patch_build(const PatchMesh &m, const std::vector<int32_t> &order, int own_size, int nu, bool backward,
-                        bool neumann, bool ring, std::vector<PatchHost> &part) {
+                        bool neumann, bool ring, std::vector<PatchHost> &part, int group_max = INT32_MAX) {
   const int nA = m.nA, np = (nA + own_size - 1) / own_size;
   part.clear();
   if (m.cptr[(nA + 63) / 64] >= (int64_t)1 << PATCH_BASE_BITS || nu < 1 || nu > 2) return false;
@@ -248,6 +256,10 @@ inline bool patch_build(const PatchMesh &m, const std::vector<int32_t> &order, i
         D.cnt[c][1] = cntg[3 * c] + (nu == 2 ? cntg[3 * c + 1] : 0);
         D.cnt[c][0] = cntg[3 * c] + cntg[3 * c + 1] + cntg[3 * c + 2];
         H.max_group = std::max(H.max_group, D.cnt[c][0]);
+      }
+      if (H.max_group > group_max) {
+        bad[t] = 1;
+        break;
       }
       D.ncs = at[15];
       D.own_e = cntg[15];

@@ -2914,6 +2914,7 @@ static int amg_capture(ufe_ctx *ctx) {
 // 800 leaves room for denser colours before the rebuild.
 constexpr size_t PATCH_LDS_MAX = 64 * 1024;
 constexpr size_t SOR_LDS_MAX = 156 * 1024;   // of the 160 KiB of a CU
+constexpr int SOR_THREADS_MAX = 1024;        // of a workgroup of the SOR loop, one row of a colour each
 constexpr int SOR_PATCH_MIN = 64;            // own points of a workgroup of the SOR loop, at least
 constexpr int PATCH_CUS = 256;               // CUs of an MI355X
 constexpr int PATCH_LARGE = 1 << 17;         // points from which the large patches fill the chip
@@ -3043,7 +3044,7 @@ static int patch_prepare(ufe_ctx *ctx, std::initializer_list<PatchKind> kinds, i
     const bool sor = k == PATCH_SOR64;
     bool fits = false;
     for (int tries = 0; tries < 6 && !fits; tries++, sh.own = sh.own * 3 / 4) {
-      if (!patch_build(m, order, sh.own, nu, k == PATCH_POST32, true, !sor, parts)) break;
+      if (!patch_build(m, order, sh.own, nu, k == PATCH_POST32, true, !sor, parts, sor ? SOR_THREADS_MAX : INT32_MAX)) break;
       int group = 0;
       S.P = PatchDev{};
       for (const PatchHost &H : parts) {
@@ -3058,7 +3059,7 @@ static int patch_prepare(ufe_ctx *ctx, std::initializer_list<PatchKind> kinds, i
       if (sor) {                       // the number of workgroups is bounded: wide enough ones or none
         sh.bs = group <= 256 ? 256 : group <= 512 ? 512 : 1024;
         S.lds = patch_sor_lds(S.P, sh.bs == 1024);
-        fits = group <= 1024 && S.lds <= SOR_LDS_MAX;
+        fits = S.lds <= SOR_LDS_MAX;
         break;
       }
       S.lds = patch_lds_bytes(S.P.cap, S.P.cap_ov);
@@ -3416,6 +3417,11 @@ static const PatchSet *sor_patches(ufe_ctx *ctx, int *err) {
     const char *off = std::getenv("UFE_SOR_PATCH");
     if (off && off[0] == '0') {
       S.built = true;
+      return nullptr;
+    }
+    const int own = patch_shape(ctx, PATCH_SOR64).own;
+    if (patch_least_group(ctx->colour_active, (ctx->nA + own - 1) / own) > SOR_THREADS_MAX) {
+      S.built = true;                // found from the colours, before anything is read back or walked
       return nullptr;
     }
     bool offered = false;
