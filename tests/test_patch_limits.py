@@ -57,3 +57,93 @@ def test_least_group_never_exceeds_the_walked_one(lib, kind, n, own, nu):
     print(f"  {kind} {n} own {own}: colours {m['active']} of {m['n']}, least {out[0]}, walked {out[1]}", flush=True)
     assert 0 < out[0] <= out[1]
     assert (out[2], out[3]) == (1, 0)
+
+
+OUT_OF_MEMORY = r"""
+#include <atomic>
+#include <cstdio>
+#include <cstdlib>
+#include <new>
+#include "patch_host.h"
+static std::atomic<long> left{1L << 40};
+void *operator new(size_t n) {
+  void *p = left.fetch_sub(1) > 0 ? std::malloc(n ? n : 1) : nullptr;
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
+using namespace ufe;
+// a grid of n x n points, coloured so that the four neighbours of a point have the other colours; its rim: edge points
+int main() {
+  const int n = 300, nA = n * n;
+  std::vector<int> id(nA), at(nA);
+  int cs[6], ca[5], k = 0;
+  auto rim = [&](int p) { return p % n == 0 || p / n == 0 || p % n == n - 1 || p / n == n - 1; };
+  for (int c = 0; c < 5; c++) {
+    cs[c] = k;
+    for (int edge = 0; edge < 2; edge++) {
+      for (int p = 0; p < nA; p++)
+        if ((p % n + 2 * (p / n)) % 5 == c && rim(p) == (edge == 1)) id[k] = p, at[p] = k++;
+      if (!edge) ca[c] = k - cs[c];
+    }
+  }
+  cs[5] = nA;
+  std::vector<int64_t> cptr((nA + 63) / 64 + 1);
+  for (size_t i = 0; i < cptr.size(); i++) cptr[i] = 256 * (int64_t)i;
+  std::vector<uint8_t> deg(nA);
+  std::vector<int32_t> col(cptr.back()), er, ep{0}, ec;
+  std::vector<uint32_t> key(nA);
+  for (int q = 0; q < nA; q++) {
+    const int p = id[q], x = p % n, y = p / n;
+    key[q] = (uint32_t)p;
+    int d = 0;
+    for (int v : {x ? p - 1 : -1, x < n - 1 ? p + 1 : -1, y ? p - n : -1, y < n - 1 ? p + n : -1})
+      if (v >= 0) col[cptr[q >> 6] + (q & 63) + 64 * d++] = at[v];
+    deg[q] = (uint8_t)d;
+    if (rim(p)) {                    // a corner of the rim averages its inner diagonal
+      er.push_back(q);
+      int inner[4], m = 0;
+      for (int j = 0; j < d; j++)
+        if (!rim(id[col[cptr[q >> 6] + (q & 63) + 64 * j]])) inner[m++] = col[cptr[q >> 6] + (q & 63) + 64 * j];
+      if (!m) inner[m++] = at[(y ? n - 2 : 1) * n + (x ? n - 2 : 1)];
+      ec.insert(ec.end(), inner, inner + m);
+      ep.push_back((int32_t)ec.size());
+    }
+  }
+  const PatchMesh m{nA, cs, ca, cptr.data(), deg.data(), col.data(), (int)er.size(), 0, er.data(), ep.data(), ec.data(),
+                    nullptr, nullptr, nullptr, key.data(), nullptr};
+  const std::vector<int32_t> order = patch_order(m);
+  int whole = 0, refused = 0;
+  for (long allow = 0; allow < 4000; allow = allow < 200 ? allow + 1 : allow + 97) {
+    std::vector<PatchHost> parts;
+    bool built = false;
+    left = allow;
+    try {
+      built = patch_build(m, order, 200, 2, false, true, true, parts);
+    } catch (const std::bad_alloc &) {   // on the calling thread: its C interface reports it
+    }
+    left = 1L << 40;
+    size_t own = 0;
+    for (const PatchHost &H : parts)
+      for (const PatchDesc &d : H.d) own += d.own[0] + d.own[1] + d.own[2] + d.own[3] + d.own[4] + d.own_e + d.own_k;
+    if (built && own != (size_t)nA) return std::printf("allowed %ld: %zu of %d points\n", allow, own, nA), 1;
+    (built ? whole : refused)++;
+  }
+  std::printf("%d whole, %d refused\n", whole, refused);
+  return whole && refused ? 0 : 2;
+}
+"""
+
+
+def test_running_out_of_host_memory_ends_the_walk_and_not_the_process(tmp_path):
+    """operator new fails after a number of allocations, on whichever thread asks."""
+    cxx = shutil.which("g++")
+    if not cxx:
+        pytest.skip("g++ not available")
+    (tmp_path / "oom.cpp").write_text(OUT_OF_MEMORY)
+    subprocess.run([cxx, "-std=c++17", "-O2", "-Wall", "-Wextra", "-pthread", f"-I{CSRC}", str(tmp_path / "oom.cpp"), "-o",
+                    str(tmp_path / "oom")], check=True)
+    r = subprocess.run([str(tmp_path / "oom")], capture_output=True, text=True, timeout=120)
+    print(r.stdout, r.stderr, flush=True)
+    assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)

@@ -5,7 +5,7 @@
 
 #include <algorithm>
 #include <cstdint>
-#include <system_error>
+#include <exception>
 #include <thread>
 #include <utility>
 #include <vector>
@@ -35,7 +35,7 @@ inline void amg_parts(int n, int parts, F body) {
     const int b = (int)((int64_t)n * t / parts), e = (int)((int64_t)n * (t + 1) / parts);
     try {
       th.emplace_back(body, t, b, e);
-    } catch (const std::system_error &) {
+    } catch (const std::exception &) {   // no thread, or no memory for one
       body(t, b, e);
     }
   }

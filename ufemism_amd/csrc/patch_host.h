@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <cstdint>
 #include <cstdlib>
+#include <new>
 #include <vector>
 
 #include "amg_host.h"
@@ -135,7 +136,9 @@ inline std::vector<int32_t> patch_order(const PatchMesh &m) {
 // rows).  Built in contiguous parts on the host's threads; the offsets in the
 // descriptors count from the start of the first part, so that the parts are
 // simply put one after another.  Returns false when the mesh does not fit the
-// packed indices, or at the first patch with more than group_max rows of a colour.
+// packed indices, at the first patch with more than group_max rows of a colour, or
+// where host memory runs out on one of the threads (an exception must not leave a
+// thread).
 inline bool patch_build(const PatchMesh &m, const std::vector<int32_t> &order, int own_size, int nu, bool backward,
                         bool neumann, bool ring, std::vector<PatchHost> &part, int group_max = INT32_MAX) {
   const int nA = m.nA, np = (nA + own_size - 1) / own_size;
@@ -159,19 +162,13 @@ inline bool patch_build(const PatchMesh &m, const std::vector<int32_t> &order, i
   const int parts = std::min(np, amg_threads(nA));
   part.resize(parts);
   std::vector<uint8_t> bad(parts, 0);
-  auto body = [&](int t, int b0, int b1) {
+  auto walk = [&](int t, int b0, int b1, uint64_t *where) {
     PatchHost &H = part[t];
     const size_t guess = (size_t)(b1 - b0) * own_size * 2;
     H.rows.reserve(guess + guess / 4);
     H.sbase.reserve(guess);
     H.ovf.reserve(guess);
     H.lcol.reserve(3 * guess);
-    // point -> (patch + 1, entry of its list); zero pages until a point is met
-    uint64_t *where = static_cast<uint64_t *>(std::calloc((size_t)nA, sizeof(uint64_t)));
-    if (!where) {
-      bad[t] = 1;
-      return;
-    }
     std::vector<int32_t> pts, pend[7], now, loc, ent;   // ent: the entries of a computed row's neighbours
     std::vector<int64_t> ent0;                          // per entry, -1: not computed
     std::vector<int8_t> sweeps;   // sweeps that compute an entry (0: only read; edge points and corners: 1)
@@ -322,9 +319,18 @@ inline bool patch_build(const PatchMesh &m, const std::vector<int32_t> &order, i
       if (neumann) H.max_ncol = std::max(H.max_ncol, H.nptr.back() - H.nptr[D.nptr]);
       H.d.push_back(D);
     }
-    std::free(where);
   };
-  amg_parts(np, parts, body);
+  amg_parts(np, parts, [&](int t, int b0, int b1) {
+    // point -> (patch + 1, entry of its list); zero pages until a point is met
+    uint64_t *where = static_cast<uint64_t *>(std::calloc((size_t)nA, sizeof(uint64_t)));
+    try {
+      if (where) walk(t, b0, b1, where);
+      else bad[t] = 1;
+    } catch (const std::bad_alloc &) {
+      bad[t] = 1;
+    }
+    std::free(where);
+  });
   size_t list = 0, comp = 0, ov = 0, nptr = 0, ncol = 0;
   for (int t = 0; t < parts; t++) {
     PatchHost &H = part[t];

@@ -2995,7 +2995,7 @@ static int patch_upload(ufe_ctx *ctx, const std::vector<PatchHost> &parts, Patch
 
 // Builds the wanted patch sets that are not there yet
 static bool sor_patch_resident(ufe_ctx *ctx, const PatchSet &S);
-static int patch_prepare(ufe_ctx *ctx, std::initializer_list<PatchKind> kinds, int nu) {
+static int patch_prepare(ufe_ctx *ctx, std::initializer_list<PatchKind> kinds, int nu) try {
   bool all = true;
   for (PatchKind k : kinds) all = all && ctx->patch[k][nu - 1].built;
   if (all) return UFE_OK;
@@ -3073,6 +3073,9 @@ static int patch_prepare(ufe_ctx *ctx, std::initializer_list<PatchKind> kinds, i
     }
     S.built = true;
   }
+  return UFE_OK;
+} catch (const std::bad_alloc &) {   // no host memory: the colour launches do without
+  for (PatchKind k : kinds) ctx->patch[k][nu - 1].built = true;
   return UFE_OK;
 }
 
