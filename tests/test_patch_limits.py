@@ -147,3 +147,69 @@ def test_running_out_of_host_memory_ends_the_walk_and_not_the_process(tmp_path):
     r = subprocess.run([str(tmp_path / "oom")], capture_output=True, text=True, timeout=120)
     print(r.stdout, r.stderr, flush=True)
     assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
+
+
+THREADS = r"""
+#include <cstdio>
+#include <cstring>
+#include "patch_host.h"
+using namespace ufe;
+extern "C" int threads_for(int64_t n) { return patch_threads(n); }
+extern "C" int same(int nA, const int *cs, const int *ca, const int64_t *cptr, const uint8_t *deg, const int32_t *col,
+                    int n_neu, const int32_t *nr, const int32_t *np_, const int32_t *nc, int n_cor, const int32_t *kr,
+                    const int32_t *kp, const int32_t *kc, const uint32_t *key, int own, int backward) {
+  const PatchMesh m{nA, cs, ca, cptr, deg, col, n_neu, n_cor, nr, np_, nc, kr, kp, kc, key, nullptr};
+  const std::vector<int32_t> order = patch_order(m);
+  PatchHost J[2];
+  for (int i = 0; i < 2; i++) {
+    std::vector<PatchHost> parts;
+    if (!patch_build(m, order, own, 2, backward != 0, true, true, parts, INT32_MAX, i ? 7 : 1)) return -1;
+    if (parts.size() != (i ? 7u : 1u)) return -2;
+    auto join = [](auto &a, auto &b) { a.insert(a.end(), b.begin(), b.end()); };
+    for (PatchHost &q : parts) {
+      join(J[i].d, q.d);
+      join(J[i].rows, q.rows);
+      join(J[i].nptr, q.nptr);
+      join(J[i].sbase, q.sbase);
+      join(J[i].lcol, q.lcol);
+      join(J[i].ov_e, q.ov_e);
+      join(J[i].ovf, q.ovf);
+      join(J[i].ov_c, q.ov_c);
+      join(J[i].ncol, q.ncol);
+    }
+  }
+  if (J[0].d.size() != J[1].d.size()) return -3;
+  for (size_t b = 0; b < J[0].d.size(); b++) {
+    const PatchDesc &x = J[0].d[b], &y = J[1].d[b];
+    auto lists = [](const PatchHost &H, const PatchDesc &d) {
+      return std::vector<int32_t>(H.rows.begin() + d.list, H.rows.begin() + d.list + d.nlist);
+    };
+    if (x.nlist != y.nlist || x.ncs != y.ncs || x.nov != y.nov || x.list != y.list || lists(J[0], x) != lists(J[1], y)) return -4;
+  }
+  return J[0].sbase == J[1].sbase && J[0].lcol == J[1].lcol && J[0].ov_e == J[1].ov_e && J[0].ovf == J[1].ovf &&
+         J[0].ov_c == J[1].ov_c;
+}
+"""
+
+
+@pytest.mark.parametrize("own,backward", [(64, 0), (240, 1)])
+def test_patches_do_not_depend_on_the_threads(tmp_path, own, backward):
+    """A mesh of 16k vertices is walked by several threads (where the machine has
+    them), with the patches of one."""
+    cxx = shutil.which("g++")
+    if not cxx:
+        pytest.skip("g++ not available")
+    (tmp_path / "threads.cpp").write_text(THREADS)
+    so = tmp_path / "threads.so"
+    subprocess.run([cxx, "-std=c++17", "-O2", "-Wall", "-Wextra", "-fPIC", "-shared", "-pthread", f"-I{CSRC}",
+                    str(tmp_path / "threads.cpp"), "-o", str(so)], check=True)
+    lib = ctypes.CDLL(str(so))
+    lib.threads_for.argtypes = [ctypes.c_int64]
+    assert lib.threads_for(200) == 1 and lib.threads_for(64000) <= lib.threads_for(1 << 22) <= 16
+    if len(os.sched_getaffinity(0)) > 1:
+        assert lib.threads_for(64000) > 1
+    m = colour_order(geometry.marine(5000, seed=8).mesh)
+    ptr = lambda a: ctypes.c_void_p(np.ascontiguousarray(a).ctypes.data)  # noqa: E731
+    assert lib.same(m["n"], ptr(m["start"]), ptr(m["active"]), ptr(m["cptr"]), ptr(m["deg"]), ptr(m["col"]),
+                    len(m["neu"][0]), *map(ptr, m["neu"]), len(m["cor"][0]), *map(ptr, m["cor"]), ptr(m["key"]), own,
+                    backward) == 1

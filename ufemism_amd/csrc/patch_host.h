@@ -60,6 +60,17 @@ struct PatchHost {                // a part of the patches, one after another
 
 constexpr int PATCH_BASE_BITS = 27;
 
+// Host threads for the patches of n points: one per 2,048 points (about a third of
+// a millisecond of walking), at most the hardware's and 16.  A mesh's first solve
+// waits for its patches, and on small meshes a solve takes no longer than a walk on
+// one thread.  First solve of a 16k-vertex mesh with the SOR loop / by multigrid
+// (the sets side by side, 16 threads): 7.3 / 38.0 -> 3.8 / 24.5 ms, where the colour
+// launches take 4.0 / 25.3.
+inline int patch_threads(int64_t n) {
+  const unsigned h = std::thread::hardware_concurrency();
+  return (int)std::max<int64_t>(1, std::min<int64_t>(n / 2048, std::min(h, 16u)));
+}
+
 // The buffers beside the patches: makes those that are not there yet, each on its
 // own, so that a call after one that stopped half-way makes the rest.  make(p)
 // returns 0, with p still null where there is no room, or an error, which ends
@@ -105,7 +116,7 @@ inline std::vector<int32_t> patch_order(const PatchMesh &m) {
   int big = 0;
   for (int r = 1; r < 6; r++)
     if (len(r) > len(big)) big = r;
-  const int parts = amg_threads(m.nA);
+  const int parts = patch_threads(m.nA);
   amg_parts(parts, parts, [&](int, int t0, int t1) {
     for (int t = t0; t < t1; t++) {
       int h[6], e[6];
@@ -138,9 +149,11 @@ inline std::vector<int32_t> patch_order(const PatchMesh &m) {
 // simply put one after another.  Returns false when the mesh does not fit the
 // packed indices, at the first patch with more than group_max rows of a colour, or
 // where host memory runs out on one of the threads (an exception must not leave a
-// thread).
+// thread).  threads: at most so many (0: patch_threads); the patches do not depend
+// on it.
 inline bool patch_build(const PatchMesh &m, const std::vector<int32_t> &order, int own_size, int nu, bool backward,
-                        bool neumann, bool ring, std::vector<PatchHost> &part, int group_max = INT32_MAX) {
+                        bool neumann, bool ring, std::vector<PatchHost> &part, int group_max = INT32_MAX,
+                        int threads = 0) {
   const int nA = m.nA, np = (nA + own_size - 1) / own_size;
   part.clear();
   if (m.cptr[(nA + 63) / 64] >= (int64_t)1 << PATCH_BASE_BITS || nu < 1 || nu > 2) return false;
@@ -159,7 +172,7 @@ inline bool patch_build(const PatchMesh &m, const std::vector<int32_t> &order, i
     const auto it = std::lower_bound(place.begin(), place.end(), std::make_pair(p, (int32_t)-1));
     return it != place.end() && it->first == p ? it->second : -1;
   };
-  const int parts = std::min(np, amg_threads(nA));
+  const int parts = std::min(np, threads > 0 ? threads : patch_threads(nA));
   part.resize(parts);
   std::vector<uint8_t> bad(parts, 0);
   auto walk = [&](int t, int b0, int b1, uint64_t *where) {
@@ -172,7 +185,7 @@ inline bool patch_build(const PatchMesh &m, const std::vector<int32_t> &order, i
     std::vector<int32_t> pts, pend[7], now, loc, ent;   // ent: the entries of a computed row's neighbours
     std::vector<int64_t> ent0;                          // per entry, -1: not computed
     std::vector<int8_t> sweeps;   // sweeps that compute an entry (0: only read; edge points and corners: 1)
-    std::vector<std::pair<int32_t, int32_t>> ownrows;
+    std::vector<uint8_t> group;
     for (int b = b0; b < b1 && !bad[t]; b++) {
       const uint64_t tag = (uint64_t)(b + 1) << 32;
       pts.clear();
@@ -242,7 +255,8 @@ inline bool patch_build(const PatchMesh &m, const std::vector<int32_t> &order, i
         return 19;
       };
       int cntg[20] = {0}, at[20];
-      for (int e = 0; e < n; e++) cntg[rank(e)]++;
+      group.resize(n);
+      for (int e = 0; e < n; e++) cntg[group[e] = (uint8_t)rank(e)]++;
       for (int g = 0, s = 0; g < 20; g++) {
         at[g] = s;
         s += cntg[g];
@@ -270,12 +284,8 @@ inline bool patch_build(const PatchMesh &m, const std::vector<int32_t> &order, i
       D.nptr = (int32_t)H.nptr.size();
       loc.resize(n);
       H.rows.resize(D.list + n);
-      // own rows in ascending order (contiguous in their colour); the others as met
-      ownrows.clear();
-      for (int e = 0; e < nown; e++) ownrows.push_back({pts[e], e});
-      std::sort(ownrows.begin(), ownrows.end());
-      for (auto &x : ownrows) loc[x.second] = at[rank(x.second)]++;
-      for (int e = nown; e < n; e++) loc[e] = at[rank(e)]++;
+      // as met: the own rows first, in ascending order inside a colour (contiguous), as the Hilbert order has them
+      for (int e = 0; e < n; e++) loc[e] = at[group[e]]++;
       std::vector<int32_t> &inv = now;   // list position -> entry
       inv.resize(n);
       for (int e = 0; e < n; e++) {

@@ -14,6 +14,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -2953,44 +2954,80 @@ static int patch_alloc(ufe_ctx *ctx, T *&p, size_t n) {
   return UFE_OK;
 }
 
-// The parts of one patch set in one device allocation (S.P.d null: no room)
+// The parts of one patch set, joined by the host's threads and copied to one device
+// allocation at once (S.P.d null: no room); a copy for each of nine arrays of 16
+// parts took longer than the walk.
 static int patch_upload(ufe_ctx *ctx, const std::vector<PatchHost> &parts, PatchSet &S) {
-  char *base = nullptr;
-  size_t total = 0;
-  int r;
-  auto put = [&](auto PatchHost::*field, auto *&dst) -> int {
-    using E = typename std::decay_t<decltype(parts[0].*field)>::value_type;
-    size_t n = 0;
-    for (const PatchHost &H : parts) n += (H.*field).size();
-    if (!base) {                     // first round: sizes only
-      total += (n * sizeof(E) + 255) / 256 * 256;
-      return UFE_OK;
-    }
-    E *d = reinterpret_cast<E *>(base + total);
-    dst = d;
-    for (const PatchHost &H : parts) {
-      const auto &v = H.*field;
-      if (!v.empty()) HIPCHK(ctx, hipMemcpyAsync(d, v.data(), v.size() * sizeof(E), hipMemcpyHostToDevice, ctx->stream));
-      d += v.size();
-    }
-    total += (n * sizeof(E) + 255) / 256 * 256;
-    return UFE_OK;
+  auto fields = [&](auto f) {
+    f(0, &PatchHost::d, S.P.d);
+    f(1, &PatchHost::rows, S.P.rows);
+    f(2, &PatchHost::nptr, S.P.nptr);
+    f(3, &PatchHost::sbase, S.P.sbase);
+    f(4, &PatchHost::lcol, S.P.lcol);
+    f(5, &PatchHost::ov_e, S.P.ov_e);
+    f(6, &PatchHost::ovf, S.P.ovf);
+    f(7, &PatchHost::ov_c, S.P.ov_c);
+    f(8, &PatchHost::ncol, S.P.ncol);
   };
-  for (int round = 0; round < 2; round++) {
-    if ((r = put(&PatchHost::d, S.P.d)) || (r = put(&PatchHost::rows, S.P.rows)) ||
-        (r = put(&PatchHost::nptr, S.P.nptr)) || (r = put(&PatchHost::sbase, S.P.sbase)) ||
-        (r = put(&PatchHost::lcol, S.P.lcol)) || (r = put(&PatchHost::ov_e, S.P.ov_e)) ||
-        (r = put(&PatchHost::ovf, S.P.ovf)) || (r = put(&PatchHost::ov_c, S.P.ov_c)) ||
-        (r = put(&PatchHost::ncol, S.P.ncol)))
-      return r;
-    if (round == 0) {
-      if ((r = patch_alloc(ctx, base, total))) return r;
-      if (!base) return UFE_OK;
-      total = 0;
-    }
-  }
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));   // the parts go with the caller
+  std::vector<size_t> first[9];      // of each array: the first byte of each part
+  size_t total = 0;
+  fields([&](int k, auto field, auto *&dst) {
+    first[k].assign(1, total);
+    for (const PatchHost &H : parts) first[k].push_back(first[k].back() + (H.*field).size() * sizeof(*dst));
+    total = (first[k].back() + 255) / 256 * 256;
+  });
+  char *base = nullptr;
+  if (const int r = patch_alloc(ctx, base, total)) return r;
+  if (!base) return UFE_OK;
+  const std::unique_ptr<char[]> host(new char[total]);
+  const int threads = (int)std::min({parts.size(), (size_t)patch_threads(ctx->nA), 1 + (total >> 20)});
+  amg_parts((int)parts.size(), threads, [&](int, int t0, int t1) {
+    for (int t = t0; t < t1; t++)
+      fields([&](int k, auto field, auto *&) {
+        const auto &v = parts[t].*field;
+        if (!v.empty()) std::memcpy(host.get() + first[k][t], v.data(), first[k][t + 1] - first[k][t]);
+      });
+  });
+  HIPCHK(ctx, hipMemcpyAsync(base, host.get(), total, hipMemcpyHostToDevice, ctx->stream));
+  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));   // the host copy goes with this call
+  fields([&](int k, auto, auto *&dst) {
+    dst = reinterpret_cast<std::remove_reference_t<decltype(dst)>>(base + first[k][0]);
+  });
   return UFE_OK;
+}
+
+// One set of patches on the host, smaller ones until they fit the workgroup (S.bs 0: none do)
+static void patch_find(const ufe_ctx *ctx, const PatchMesh &m, const std::vector<int32_t> &order, PatchKind k, int nu,
+                       int threads, std::vector<PatchHost> &parts, PatchSet &S) {
+  PatchShape sh = patch_shape(ctx, k);
+  const bool sor = k == PATCH_SOR64;
+  bool fits = false;
+  for (int tries = 0; tries < 6 && !fits; tries++, sh.own = sh.own * 3 / 4) {
+    if (!patch_build(m, order, sh.own, nu, k == PATCH_POST32, true, !sor, parts, sor ? SOR_THREADS_MAX : INT32_MAX,
+                     threads))
+      break;
+    int group = 0;
+    S.P = PatchDev{};
+    for (const PatchHost &H : parts) {
+      group = std::max(group, H.max_group);
+      S.P.np += (int)H.d.size();
+      S.P.cap = std::max(S.P.cap, H.max_list);
+      S.P.cap_ov = std::max(S.P.cap_ov, H.max_ov);
+      S.P.cap_ncs = std::max(S.P.cap_ncs, H.max_ncs);
+      S.P.cap_neu = std::max(S.P.cap_neu, H.max_neu);
+      S.P.cap_ncol = std::max(S.P.cap_ncol, H.max_ncol);
+    }
+    if (sor) {                         // the number of workgroups is bounded: wide enough ones or none
+      sh.bs = group <= 256 ? 256 : group <= 512 ? 512 : SOR_THREADS_MAX;
+      S.lds = patch_sor_lds(S.P, sh.bs == SOR_THREADS_MAX);
+      fits = S.lds <= SOR_LDS_MAX;
+      break;
+    }
+    S.lds = patch_lds_bytes(S.P.cap, S.P.cap_ov);
+    fits = group <= sh.bs && S.lds <= PATCH_LDS_MAX;
+  }
+  S.bs = fits ? sh.bs : 0;
+  if (fits && sor) patch_mark_shared(ctx->nA, parts);
 }
 
 // Builds the wanted patch sets that are not there yet
@@ -3035,41 +3072,28 @@ static int patch_prepare(ufe_ctx *ctx, std::initializer_list<PatchKind> kinds, i
     if (d_place) HIPCHK(ctx, hipMemcpy(d_place, place.data(), sizeof(int32_t) * nA, hipMemcpyHostToDevice));
     ctx->d_place = d_place;
   }
-  for (PatchKind k : kinds) {
-    PatchSet &S = ctx->patch[k][nu - 1];
-    if (S.built) continue;
-    PatchShape sh = patch_shape(ctx, k);
-    ctx->paths.patch_sets++;
-    std::vector<PatchHost> parts;
-    const bool sor = k == PATCH_SOR64;
-    bool fits = false;
-    for (int tries = 0; tries < 6 && !fits; tries++, sh.own = sh.own * 3 / 4) {
-      if (!patch_build(m, order, sh.own, nu, k == PATCH_POST32, true, !sor, parts, sor ? SOR_THREADS_MAX : INT32_MAX)) break;
-      int group = 0;
-      S.P = PatchDev{};
-      for (const PatchHost &H : parts) {
-        group = std::max(group, H.max_group);
-        S.P.np += (int)H.d.size();
-        S.P.cap = std::max(S.P.cap, H.max_list);
-        S.P.cap_ov = std::max(S.P.cap_ov, H.max_ov);
-        S.P.cap_ncs = std::max(S.P.cap_ncs, H.max_ncs);
-        S.P.cap_neu = std::max(S.P.cap_neu, H.max_neu);
-        S.P.cap_ncol = std::max(S.P.cap_ncol, H.max_ncol);
+  // the sets are walked side by side, each by its share of the threads
+  std::vector<PatchKind> todo;
+  for (PatchKind k : kinds)
+    if (!ctx->patch[k][nu - 1].built) todo.push_back(k);
+  std::vector<std::vector<PatchHost>> parts(todo.size());
+  const int threads = patch_threads(nA), nk = (int)todo.size(), each = std::max(1, threads / nk);
+  amg_parts(nk, std::min(nk, threads), [&](int, int i0, int i1) {
+    for (int i = i0; i < i1; i++) {
+      PatchSet &S = ctx->patch[todo[i]][nu - 1];
+      try {
+        patch_find(ctx, m, order, todo[i], nu, each, parts[i], S);
+      } catch (const std::bad_alloc &) {
+        S.bs = 0;
       }
-      if (sor) {                       // the number of workgroups is bounded: wide enough ones or none
-        sh.bs = group <= 256 ? 256 : group <= 512 ? 512 : 1024;
-        S.lds = patch_sor_lds(S.P, sh.bs == 1024);
-        fits = S.lds <= SOR_LDS_MAX;
-        break;
-      }
-      S.lds = patch_lds_bytes(S.P.cap, S.P.cap_ov);
-      fits = group <= sh.bs && S.lds <= PATCH_LDS_MAX;
     }
-    if (fits) {
-      if (sor) patch_mark_shared(nA, parts);
-      if ((r = patch_upload(ctx, parts, S))) return r;
-      S.bs = sh.bs;
-      S.ok = S.P.d && (!sor || sor_patch_resident(ctx, S));
+  });
+  for (int i = 0; i < nk; i++) {
+    PatchSet &S = ctx->patch[todo[i]][nu - 1];
+    ctx->paths.patch_sets++;
+    if (S.bs) {
+      if ((r = patch_upload(ctx, parts[i], S))) return r;
+      S.ok = S.P.d && (todo[i] != PATCH_SOR64 || sor_patch_resident(ctx, S));
     }
     S.built = true;
   }
