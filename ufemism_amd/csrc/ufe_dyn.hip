@@ -367,9 +367,15 @@ static inline int nblk(int64_t n, int b = BLOCK) { return (int)((n + b - 1) / b)
 constexpr int PROF_EVERY = 8;     // colour launches per timed sample
 // grid for XCD-major kernels: a multiple of the 8 XCDs
 static inline int xcd_grid(int64_t n) { return (nblk(n) + 7) / 8 * 8; }
-// grid of a layered kernel: points, groups of LAYERS layers, fields
-static inline dim3 layer_grid(int64_t n, int nz, int fields = 1) {
-  return dim3(xcd_grid(n), std::min((nz + LAYERS - 1) / LAYERS, 65535), fields);
+// grid of a layered kernel: points, groups of G layers, fields
+static inline dim3 layer_grid(int64_t n, int nz, int G, int fields = 1) {
+  return dim3(xcd_grid(n), std::min((nz + G - 1) / G, 65535), fields);
+}
+// a layered kernel's launch f(width, grid) with the width for n points
+template <typename F>
+static inline void layered(int64_t n, int nz, int fields, F f) {
+  if (nz <= 2 || n * nz <= LAYER_VALUES) f(std::integral_constant<int, 1>{}, layer_grid(n, nz, 1, fields));
+  else f(std::integral_constant<int, LAYERS>{}, layer_grid(n, nz, LAYERS, fields));
 }
 
 template <typename T>
@@ -1205,7 +1211,7 @@ int ufe_remap_build(ufe_ctx *dst, ufe_ctx *src, const ufe_mesh_geometry_desc *gs
   HIPCHK(dst, s.alloc((void **)&dd, sizeof(double) * nVd));
   k_fill<double><<<nblk(nVs), BLOCK, 0, q>>>(ones, nVs, 1.0);
   k_deriv_Aa<<<nblk(nVs), BLOCK, 0, q>>>(aa_mesh(src), ones, dx, dy);
-  k_rm_apply_cons<true><<<layer_grid(nVd, 1), BLOCK, 0, q>>>(nVd, nVs, 1, dst->d_rm_st, dst->d_rm_en, dst->d_rm_vi, dst->d_rm_w0,
+  k_rm_apply_cons<1, true><<<layer_grid(nVd, 1, 1), BLOCK, 0, q>>>(nVd, nVs, 1, dst->d_rm_st, dst->d_rm_en, dst->d_rm_vi, dst->d_rm_w0,
                                               dst->d_rm_w1x, dst->d_rm_w1y, ones, dx, dy, dd);
   LAUNCHCHK(dst);
   std::vector<double> hd(nVd);
@@ -1295,15 +1301,21 @@ int ufe_remap_field(ufe_ctx *dst, ufe_ctx *src, int method, const double *d_src,
   const int nVs = dst->rm_nVs, nVd = dst->rm_nVd;
   switch (method) {
     case UFE_REMAP_TRILIN:
-      k_rm_apply_trilin<<<layer_grid(nVd, nz), BLOCK, 0, q>>>(nVd, nVs, nz, dst->d_rm_tvi, dst->d_rm_tw, d_src, d_dst);
+      layered(nVd, nz, 1, [&](auto G, dim3 grid) {
+        k_rm_apply_trilin<G.value><<<grid, BLOCK, 0, q>>>(nVd, nVs, nz, dst->d_rm_tvi, dst->d_rm_tw, d_src, d_dst);
+      });
       break;
     case UFE_REMAP_NEAREST_NEIGHBOUR:
-      k_rm_apply_nn<<<layer_grid(nVd, nz), BLOCK, 0, q>>>(nVd, nVs, nz, dst->d_rm_nn, d_src, d_dst);
+      layered(nVd, nz, 1, [&](auto G, dim3 grid) {
+        k_rm_apply_nn<G.value><<<grid, BLOCK, 0, q>>>(nVd, nVs, nz, dst->d_rm_nn, d_src, d_dst);
+      });
       break;
     case UFE_REMAP_CONS_1ST_ORDER:
-      k_rm_apply_cons<false><<<layer_grid(nVd, nz), BLOCK, 0, q>>>(nVd, nVs, nz, dst->d_rm_st, dst->d_rm_en, dst->d_rm_vi,
-                                                                   dst->d_rm_w0, nullptr, nullptr, d_src, nullptr,
-                                                                   nullptr, d_dst);
+      layered(nVd, nz, 1, [&](auto G, dim3 grid) {
+        k_rm_apply_cons<G.value, false><<<grid, BLOCK, 0, q>>>(nVd, nVs, nz, dst->d_rm_st, dst->d_rm_en, dst->d_rm_vi,
+                                                               dst->d_rm_w0, nullptr, nullptr, d_src, nullptr, nullptr,
+                                                               d_dst);
+      });
       break;
     case UFE_REMAP_CONS_2ND_ORDER: {
       // the derivatives' space is kept until the mesh goes (allocating and
@@ -1317,10 +1329,14 @@ int ufe_remap_field(ufe_ctx *dst, ufe_ctx *src, int method, const double *d_src,
         dst->rm_work_len = need;
       }
       double *dx = dst->rm_work, *dy = dx + (size_t)nVs * nz;
-      k_deriv_Aa_3D<<<layer_grid(nVs, nz), BLOCK, 0, q>>>(aa_mesh(src), nz, d_src, dx, dy);
-      k_rm_apply_cons<true><<<layer_grid(nVd, nz), BLOCK, 0, q>>>(nVd, nVs, nz, dst->d_rm_st, dst->d_rm_en, dst->d_rm_vi,
-                                                                  dst->d_rm_w0, dst->d_rm_w1x, dst->d_rm_w1y, d_src, dx,
-                                                                  dy, d_dst);
+      layered(nVs, nz, 1, [&](auto G, dim3 grid) {
+        k_deriv_Aa_3D<G.value><<<grid, BLOCK, 0, q>>>(aa_mesh(src), nz, d_src, dx, dy);
+      });
+      layered(nVd, nz, 1, [&](auto G, dim3 grid) {
+        k_rm_apply_cons<G.value, true><<<grid, BLOCK, 0, q>>>(nVd, nVs, nz, dst->d_rm_st, dst->d_rm_en, dst->d_rm_vi,
+                                                              dst->d_rm_w0, dst->d_rm_w1x, dst->d_rm_w1y, d_src, dx, dy,
+                                                              d_dst);
+      });
       break;
     }
     default:
@@ -1972,7 +1988,9 @@ int ufe_solve_SIA(ufe_ctx *ctx) {
 // apply_Neumann_boundary_3D of one or two fields
 static void neumann_Aa(ufe_ctx *ctx, int nz, double *d0, double *d1 = nullptr) {
   const int fields = d1 ? 2 : 1;
-  k_neumann_Aa_edges<<<layer_grid(ctx->nV, nz, fields), BLOCK, 0, ctx->stream>>>(aa_mesh(ctx), nz, d0, d1);
+  layered(ctx->nV, nz, fields, [&](auto G, dim3 grid) {
+    k_neumann_Aa_edges<G.value><<<grid, BLOCK, 0, ctx->stream>>>(aa_mesh(ctx), nz, d0, d1);
+  });
   k_neumann_Aa_corners<<<dim3(nblk(nz, 64), fields), 64, 0, ctx->stream>>>(aa_mesh(ctx), nz, d0, d1);
 }
 
@@ -5100,7 +5118,9 @@ int ufe_op_curvatures_Aa(ufe_ctx *ctx, const double *d, double *a, double *b, do
 }
 int ufe_op_derivatives_Aa_3D(ufe_ctx *ctx, const double *d, double *ddx, double *ddy, int nz) {
   NEED_MESH(ctx);
-  k_deriv_Aa_3D<<<layer_grid(ctx->nV, nz), BLOCK, 0, ctx->stream>>>(aa_mesh(ctx), nz, d, ddx, ddy);
+  layered(ctx->nV, nz, 1, [&](auto G, dim3 grid) {
+    k_deriv_Aa_3D<G.value><<<grid, BLOCK, 0, ctx->stream>>>(aa_mesh(ctx), nz, d, ddx, ddy);
+  });
   LAUNCHCHK(ctx);
   return ufe_synchronize(ctx);
 }
@@ -5117,8 +5137,9 @@ int ufe_op_upwind_derivatives_3D(ufe_ctx *ctx, const double *U, const double *V,
   if (!U || !V || !d || !ddx || !ddy || nz < 1) return UFE_BAD_INPUT;
   hipStream_t q = ctx->stream;
   HIPCHK(ctx, hipMemsetAsync(ctx->d_icount, 0, sizeof(int32_t), q));
-  k_upwind_3D<<<layer_grid(ctx->nV, nz), BLOCK, 0, q>>>(aa_mesh(ctx), tri_mesh(ctx), nz, U, V, d, ddx, ddy,
-                                                            ctx->d_icount);
+  layered(ctx->nV, nz, 1, [&](auto G, dim3 grid) {
+    k_upwind_3D<G.value><<<grid, BLOCK, 0, q>>>(aa_mesh(ctx), tri_mesh(ctx), nz, U, V, d, ddx, ddy, ctx->d_icount);
+  });
   LAUNCHCHK(ctx);
   int32_t h = 0;
   HIPCHK(ctx, hipMemcpyAsync(&h, ctx->d_icount, sizeof(int32_t), hipMemcpyDeviceToHost, q));
@@ -5159,14 +5180,16 @@ int ufe_op_neumann_AaAc(ufe_ctx *ctx, double *d) {
 int ufe_op_map_Aa_to_Ac(ufe_ctx *ctx, const double *a, double *b) { return ufe_op_map_Aa_to_Ac_3D(ctx, a, b, 1); }
 int ufe_op_map_Aa_to_Ac_3D(ufe_ctx *ctx, const double *a, double *b, int nz) {
   NEED_MESH(ctx);
-  k_map_Aa_to_Ac<<<layer_grid(ctx->nAc, nz), BLOCK, 0, ctx->stream>>>(ac_mesh(ctx), nz, a, b);
+  layered(ctx->nAc, nz, 1, [&](auto G, dim3 grid) {
+    k_map_Aa_to_Ac<G.value><<<grid, BLOCK, 0, ctx->stream>>>(ac_mesh(ctx), nz, a, b);
+  });
   LAUNCHCHK(ctx);
   return ufe_synchronize(ctx);
 }
 int ufe_op_map_Ac_to_Aa(ufe_ctx *ctx, const double *a, double *b) { return ufe_op_map_Ac_to_Aa_3D(ctx, a, b, 1); }
 int ufe_op_map_Ac_to_Aa_3D(ufe_ctx *ctx, const double *a, double *b, int nz) {
   NEED_MESH(ctx);
-  k_map_Ac_to_Aa<<<layer_grid(ctx->nV, nz), BLOCK, 0, ctx->stream>>>(aa_mesh(ctx), ctx->nAc, nz, a, b);
+  k_map_Ac_to_Aa<<<layer_grid(ctx->nV, nz, 1), BLOCK, 0, ctx->stream>>>(aa_mesh(ctx), ctx->nAc, nz, a, b);
   LAUNCHCHK(ctx);
   return ufe_synchronize(ctx);
 }
