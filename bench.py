@@ -224,6 +224,7 @@ def main():
         if mark:
             marker()
         ctx.profile_read()
+        ways = ctx.path_counts()
         ctx.profile_enable(True)
         ctx.synchronize()
         ta = time.perf_counter()
@@ -238,7 +239,9 @@ def main():
         ctx.profile_enable(False)
         prof = ctx.profile_read()
         sol = (ctx.get("U_SSA_AaAc"), ctx.get("V_SSA_AaAc"))
+        ways = {k: v - ways[k] for k, v in ctx.path_counts().items()}
         res = dict(seconds_per_solve=el / steps, sweeps_per_solve=last.sweeps,
+                   smoothing_on_patches=ways["smooth_patch"] > 0 and ways["smooth_colour"] == 0,
                    matvecs_per_solve=last.matvecs, refinements=last.refinements,
                    rel_residual=last.rel_residual, converged=last.status == 0,
                    raw_Mvertex_sweeps_per_s=nA * sweeps / el / 1e6,
@@ -296,7 +299,7 @@ def main():
                                                         "velocity_error": verr(sol)}
     R = paths[head]
     kname = {"mixed_gmres": "k_sor_colour_f32"}.get(head, "k_sor_colour")
-    if head == "mixed_gmres" and args.pc == "multigrid":
+    if head == "mixed_gmres" and R["smoothing_on_patches"]:
         kname = "k_patch_smooth"        # both smoothings: precond_sweeps sweeps and A z per launch
     elif head == "mixed_gmres" and tuning:
         kname = f"k_sor_colour_f32_tuned<{tuning['threads_per_block']},{tuning['schedule']},{tuning['loads']}>"
@@ -441,9 +444,9 @@ def bench_rows(args, ctx, step, wl, remap_wls, reps=10):
     row("ice_physical_properties", timed(lambda: ctx.ice_physical_properties(1)),
         nV * (40 * nZ + 20) + nAc * (32 * nZ + 20))
     ctx.solve_SIA()
-    # U_3D/V_3D: 5 Aa fields + A_flow in, U_3D/V_3D out; W_3D: 6 Aa fields, Nx/Ny, own and
-    # neighbour U_3D/V_3D per layer in, W_3D out
-    sia3d = nV * ((24 * nZ + 44) + (56 + 20 * (n + 1) + 16 * (n + 1) * nZ + 8 * nZ))
+    # U_3D/V_3D: 5 Aa fields + A_flow in, U_3D/V_3D out; W_3D: 6 Aa fields, Nx/Ny, U_3D/V_3D
+    # (each value once, however many neighbours gather it) in, W_3D out
+    sia3d = nV * ((24 * nZ + 44) + (56 + 20 * (n + 1) + 16 * nZ + 8 * nZ))
     row("solve_SIA_3D", timed(ctx.solve_SIA_3D), sia3d)
     # per Ac point: D_SIA_Ac, Aci, both vertices' V, U_SSA, V_SSA; per vertex: A, U_SSA, V_SSA, U_3D, V_3D
     row("critical_timesteps", timed(ctx.critical_timesteps), nAc * 80 + nV * (24 + 16 * nZ),

@@ -229,7 +229,9 @@ typedef struct ufe_linsolve_stats {
 
 /* Live kernel timing: start/stop events attached to the dispatch of every
  * 8th SOR colour-kernel launch (hipExtLaunchKernelGGL), i.e. the kernel's own
- * execution time on the library's stream. */
+ * execution time on the library's stream.  Where the multigrid smoothing runs on
+ * patches, its launches count instead: all sweeps of a smoothing in one, with the
+ * bytes that one launch needs (each input once). */
 typedef struct ufe_kernel_profile {
   int64_t launches;                 /* colour-kernel launches timed (the sample) */
   double seconds;                   /* summed event time of those launches */

@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 from ufemism_amd import abi, geometry
-from ufemism_amd.dynamics import Step
+from ufemism_amd.dynamics import Step, frozen_ssa_system
 
 pytestmark = pytest.mark.gpu
 FIELDS = ("U_SSA", "V_SSA", "Ux_SSA_Ac", "Uy_SSA_Ac", "Hi")
@@ -87,7 +87,7 @@ sys.modules["torch"] = None          # the HIP runtime the library is linked wit
 sys.path.insert(0, sys.argv[1])
 import numpy as np
 from ufemism_amd import abi, geometry
-from ufemism_amd.dynamics import Step
+from ufemism_amd.dynamics import Step, frozen_ssa_system
 for n in (300, 2000):
     ctx = abi.Context(0)
     out = Step(ctx, geometry.dome(n, seed=5, picard=3)).run()
@@ -121,3 +121,25 @@ def test_mesh_too_large_for_the_loop_is_not_walked():
     wl.params.SSA_max_inner_loops = 2
     _, c = _sor_step(wl)
     assert c["patch_sets"] == c["sor_patch"] == 0 and c["sor_colour"] > 0, c
+
+
+def test_profiled_bytes_of_a_smoothing_are_those_of_one_launch():
+    """Two sweeps in one launch read the coefficients once: the bytes it is credited
+    with stay below one colour sweep's and the residual's, and the rows are both sweeps'."""
+    print("[patch profile]", flush=True)
+    wl = geometry.marine(6000, seed=5, picard=2)
+    ctx = abi.Context(0)
+    try:
+        frozen_ssa_system(ctx, wl, picard=2)
+        ctx.profile_read()
+        ctx.profile_enable(True)
+        ctx.ssa_linear_solve(1e-6, 1000, precision=abi.UFE_MIXED, gmres=20, precond_sweeps=2, orth_passes=1,
+                             precond_type=abi.UFE_PRECOND_MULTIGRID)
+        ctx.profile_enable(False)
+        p, sweep = ctx.profile_read(), ctx.sweep_bytes()
+        assert ctx.path_counts()["smooth_patch"] > 0 and p.launches > 0
+        per = p.algorithmic_bytes / p.launches
+        assert p.rows == 2 * sweep["rows"] * p.launches
+        assert 0.5 * sweep["fp32"] < per <= sweep["fp32"] + 8 * sweep["rows"], (per, sweep)
+    finally:
+        ctx.close()

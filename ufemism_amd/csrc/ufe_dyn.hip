@@ -3150,12 +3150,13 @@ static void patch_smooth_launch(ufe_ctx *ctx, bool post, float omega, const floa
   const PatchSet &S = ctx->patch[post ? PATCH_POST32 : PATCH_PRE32][NU - 1];
   const dim3 grid((S.P.np + 7) / 8 * 8), block(BS);
   const uint8_t *skip = ctx->gl_active ? ctx->d_skip : nullptr;
-  double bytes = 0.0;
+  // what the launch cannot do without, whatever the number of sweeps: per row the
+  // coefficients with their 16-bit columns, the row's index and position, centre,
+  // Sxy and right-hand side, z out, z in (post) and the residual or A z
   int64_t rows = 0;
-  for (int c = 0; c < 5; c++) {
-    bytes += NU * ctx->bytes32[c];
-    rows += (int64_t)NU * ctx->colour_active[c];
-  }
+  for (int c = 0; c < 5; c++) rows += ctx->colour_active[c];
+  const double bytes = 10.0 * ctx->degsum + (double)rows * (36.0 + (post ? 8.0 : 0.0) + (y ? 8.0 : 0.0));
+  rows *= NU;                        // the rate counts vertex-sweeps
   const float2 *cU = ctx->d_cU32, *EV = ctx->d_EV32;
   const float *Sxy = ctx->d_Sxy32;
   if (!post)
