@@ -7,7 +7,7 @@ import sys
 import numpy as np
 import pytest
 
-from ufemism_amd import abi, geometry
+from ufemism_amd import abi, batch, geometry
 from ufemism_amd.dynamics import Step, frozen_ssa_system
 
 pytestmark = pytest.mark.gpu
@@ -86,7 +86,7 @@ import sys
 sys.modules["torch"] = None          # the HIP runtime the library is linked with
 sys.path.insert(0, sys.argv[1])
 import numpy as np
-from ufemism_amd import abi, geometry
+from ufemism_amd import abi, batch, geometry
 from ufemism_amd.dynamics import Step, frozen_ssa_system
 for n in (300, 2000):
     ctx = abi.Context(0)
@@ -143,3 +143,77 @@ def test_profiled_bytes_of_a_smoothing_are_those_of_one_launch():
         assert 0.5 * sweep["fp32"] < per <= sweep["fp32"] + 8 * sweep["rows"], (per, sweep)
     finally:
         ctx.close()
+
+
+SMOOTH = {"0": ("smooth_colour", "smooth_patch"), "1": ("smooth_patch", "smooth_colour")}
+
+
+@pytest.mark.parametrize("on", ["0", "1"])
+@pytest.mark.parametrize("kind,n,nu", [("dome", 300, 2), ("marine", 20000, 1), ("marine", 90000, 2)])
+def test_switch_of_the_smoothing_decides_the_way(kind, n, nu, on):
+    """The comparisons of the two ways compare two ways."""
+    print(f"[patch ways] {kind} {n} nu {nu} {on}", flush=True)
+    wl = getattr(geometry, kind)(n, seed=5, picard=2)
+    os.environ["UFE_AMG_PATCH"] = on
+    ctx = abi.Context(0)
+    try:
+        Step(ctx, wl)
+        ctx.set_params(wl.params, abi.UFE_MIXED, linear_rel_tol=1e-6, precond_type=abi.UFE_PRECOND_MULTIGRID,
+                       precond_sweeps=nu)
+        ctx.update_general_ice_model_data()
+        ctx.solve_SIA()
+        ctx.solve_SSA()
+        c = ctx.path_counts()
+        taken, other = SMOOTH[on]
+        assert c[taken] > 0 and c[other] == 0 and c["patch_sets"] == 2 * int(on), c
+    finally:
+        ctx.close()
+        os.environ.pop("UFE_AMG_PATCH", None)
+
+
+@pytest.mark.parametrize("on", ["0", "1"])
+def test_switch_of_the_smoothing_decides_the_way_of_a_batch(on):
+    os.environ["UFE_AMG_PATCH"] = on
+    ctx = abi.Context(0)
+    try:
+        b = batch.Batch(ctx, batch.ensemble(n=3, nv_min=1500, nv_max=4000, seed=7, picard=2))
+        ctx.update_general_ice_model_data()
+        ctx.batch_solve_SSA(2, rel_tol=1e-6, gmres_restart=20, precond_sweeps=2, precond_type=abi.UFE_PRECOND_MULTIGRID)
+        c = ctx.path_counts()
+        taken, other = SMOOTH[on]
+        assert c[taken] > 0 and c[other] == 0, c
+        del b
+    finally:
+        ctx.close()
+        os.environ.pop("UFE_AMG_PATCH", None)
+
+
+@pytest.mark.parametrize("sweep_batch", [0, 3])
+def test_unstable_solve_is_reset_on_both_ways(sweep_batch):
+    """Over-relaxation by 2.6 diverges: the first solve resets the velocities, the
+    second ends the call, with the same sweeps and the same velocities left."""
+    print(f"[sor ways] divergent, sweep batch {sweep_batch}", flush=True)
+    wl = geometry.marine(2000, seed=5, picard=5)
+    wl.params.SSA_SOR_omega = 2.6
+    wl.params.SSA_max_inner_loops = 2000
+    out = {}
+    for on in ("0", "1"):
+        os.environ["UFE_SOR_PATCH"] = on
+        ctx = abi.Context(0)
+        try:
+            Step(ctx, wl, sweep_batch=sweep_batch)
+            ctx.update_general_ice_model_data()
+            ctx.solve_SIA()
+            st = ctx.solve_SSA(allow=(abi.UFE_OK, abi.UFE_SOR_NOT_CONVERGED, abi.UFE_SSA_UNSTABLE))
+            assert st.resets == 2 and st.status == abi.UFE_SSA_UNSTABLE, (st.resets, st.status)
+            assert st.last_max_residual > 1e6
+            c = ctx.path_counts()
+            assert (c["sor_patch"] > 0, c["sor_colour"] > 0) == ((False, True) if on == "0" else (True, False)), c
+            out[on] = (list(st.sweeps)[:st.picard_iterations], st.last_max_residual,
+                       [ctx.get(k) for k in ("U_SSA", "V_SSA", "Ux_SSA_Ac", "Uy_SSA_Ac")])
+        finally:
+            ctx.close()
+            os.environ.pop("UFE_SOR_PATCH", None)
+    assert out["0"][:2] == out["1"][:2], (out["0"][:2], out["1"][:2])
+    for a, b in zip(out["0"][2], out["1"][2]):
+        assert np.array_equal(a, b)
