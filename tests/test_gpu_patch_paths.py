@@ -217,3 +217,38 @@ def test_unstable_solve_is_reset_on_both_ways(sweep_batch):
     assert out["0"][:2] == out["1"][:2], (out["0"][:2], out["1"][:2])
     for a, b in zip(out["0"][2], out["1"][2]):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("gl", [False, True])
+def test_adjoint_folds_in_one_launch_and_in_several(gl):
+    """The folds of meshes with many edge points (UFE_FOLD_MAX=0) against the one
+    workgroup of the others and against the colour launches: the same gradients."""
+    torch = pytest.importorskip("torch")
+    from ufemism_amd.adjoint import AdjointOptions, SSAProblem, ssa_velocities
+    print(f"[adjoint folds] gl {gl}", flush=True)
+    wl = geometry.marine(6000, seed=5, picard=2)
+    wl.params.use_analytical_GL_flux = gl
+    out = {}
+    for name, env in (("colours", {"UFE_AMG_PATCH": "0"}), ("one", {}), ("several", {"UFE_FOLD_MAX": "0"})):
+        os.environ.update(env)
+        ctx = abi.Context(0)
+        try:
+            step = Step(ctx, wl)
+            ctx.update_general_ice_model_data()
+            prob = SSAProblem(ctx, AdjointOptions(picard_iterations=2, lin_rel_tol=1e-10, gmres_restart=20,
+                                                  precond_sweeps=2, precond_type=abi.UFE_PRECOND_MULTIGRID))
+            tau = torch.tensor(wl.tau_c_override(step.ma["VAaAc"]), dtype=torch.float64, device=prob.dev)
+            lt = torch.log(tau).requires_grad_(True)
+            A = torch.full_like(tau, wl.A_flow).requires_grad_(True)
+            U, V = ssa_velocities(lt, A, prob)
+            (U * U + 2.0 * V * V).sum().backward()
+            out[name] = (lt.grad.clone(), A.grad.clone())
+            c = ctx.path_counts()
+            assert (c["smooth_T_patch"] > 0, c["smooth_T_colour"] > 0) == ((False, True) if name == "colours" else (True, False)), c
+        finally:
+            ctx.close()
+            for k in env:
+                os.environ.pop(k, None)
+    for name in ("one", "several"):
+        for a, b in zip(out["colours"], out[name]):
+            assert torch.equal(a, b) and float(a.abs().max()) > 0, name

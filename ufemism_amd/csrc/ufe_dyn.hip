@@ -317,6 +317,7 @@ struct ufe_ctx {
   int amg_graph_T_nu = 0;
   double2 *amg_y64 = nullptr;       // FP64 fine-level A z (adjoint)
   double2 *amg_zt64 = nullptr;      // fine vector between the transposed smoothings (patches)
+  int fold_max = FOLD_MAX;          // edge points and corners up to which one launch folds (UFE_FOLD_MAX)
   bool cor_apart = false;           // no two corners average the same point, none another corner
   float2 *amg_v32 = nullptr, *amg_z32 = nullptr;   // FP32 copies around an FP64 Krylov method
   float2 *amg_zt = nullptr, *amg_zu = nullptr;     // fine vector between the smoothings (patches)
@@ -3279,7 +3280,7 @@ static void patch_smooth_T(ufe_ctx *ctx, const AaAcMesh &mT, bool post, double o
   go(ctx, mT, post, omega, v, zin, z, y);
   const uint8_t *skip = ctx->gl_active ? ctx->d_skip : nullptr;
   const NeumannList E = neu_list(ctx), K = cor_list(ctx);
-  if (E.n + K.n <= FOLD_MAX) {
+  if (E.n + K.n <= ctx->fold_max) {
     k_fold_T<<<1, FOLD_THREADS, 0, ctx->stream>>>(mT, E, K, rev_list(ctx), skip, z, y, ctx->cor_apart ? 1 : 0);
     return;
   }
@@ -4433,6 +4434,8 @@ static int adj_solve(ufe_ctx *ctx, double tol, int m, int ks, double omega, int 
     if ((r = amg_setup(ctx))) return r;
     ctx->amg_nu = ks;
     if ((r = amg_patches(ctx))) return r;
+    const char *fold = std::getenv("UFE_FOLD_MAX");
+    ctx->fold_max = fold && *fold ? (int)std::strtol(fold, nullptr, 10) : FOLD_MAX;
     if (amg_on_patches(ctx) && !ctx->amg_zt64 && (r = patch_alloc(ctx, ctx->amg_zt64, (size_t)n))) return r;
     ctx->amg_T = true;
     k_to_f32_pair<<<nblk(n), BLOCK, 0, ctx->stream>>>(n, ctx->d_pair[1], ctx->d_EV32);
