@@ -64,8 +64,8 @@ constexpr int PATCH_BASE_BITS = 27;
 // a millisecond of walking), at most the hardware's and 16.  A mesh's first solve
 // waits for its patches, and on small meshes a solve takes no longer than a walk on
 // one thread.  First solve of a 16k-vertex mesh with the SOR loop / by multigrid
-// (the sets side by side, 16 threads): 7.3 / 38.0 -> 3.8 / 24.5 ms, where the colour
-// launches take 4.0 / 25.3.
+// (the sets side by side beside the multigrid set-up): one thread 7.3 / 38.0 ms, 16
+// 3.6 / 21.1, where the colour launches take 4.0 / 25.0.
 inline int patch_threads(int64_t n) {
   const unsigned h = std::thread::hardware_concurrency();
   return (int)std::max<int64_t>(1, std::min<int64_t>(n / 2048, std::min(h, 16u)));

@@ -17,6 +17,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "ufe_internal.h"
@@ -2419,24 +2420,18 @@ static int amg_tail_images(ufe_ctx *ctx) {
   return UFE_OK;
 }
 
-static int amg_setup(ufe_ctx *ctx) {
-  if (ctx->amg_ready) return UFE_OK;
-  const auto t0 = std::chrono::steady_clock::now();
+// The colour-ordered neighbour lists on the host, read back once for the multigrid
+// set-up and the patches (empty: not read)
+struct HostLists {
+  std::vector<int64_t> cptr;
+  std::vector<uint8_t> deg;
+  std::vector<int32_t> col, nrow, nptr, ncol, crow, cptr2, ccol;   // neighbours; edge points; corners
+};
+static int host_lists(ufe_ctx *ctx, HostLists &L) {
+  if (!L.cptr.empty()) return UFE_OK;
   const int nA = ctx->nA, nchunk = (nA + SELL - 1) / SELL;
   int r;
-  // the fine operator, read back from the device
-  std::vector<int64_t> cptr(nchunk + 1);
-  std::vector<uint8_t> deg(nA);
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  HIPCHK(ctx, hipMemcpy(cptr.data(), ctx->d_chunk_ptr, sizeof(int64_t) * (nchunk + 1), hipMemcpyDeviceToHost));
-  HIPCHK(ctx, hipMemcpy(deg.data(), ctx->d_deg, nA, hipMemcpyDeviceToHost));
-  const int64_t ne = cptr[nchunk];
-  std::vector<int32_t> col(ne);
-  std::vector<double2> cU(ne);
-  std::vector<double> Sxy(nA);
-  HIPCHK(ctx, hipMemcpy(col.data(), ctx->d_col, sizeof(int32_t) * ne, hipMemcpyDeviceToHost));
-  HIPCHK(ctx, hipMemcpy(cU.data(), ctx->d_cU, sizeof(double2) * ne, hipMemcpyDeviceToHost));
-  HIPCHK(ctx, hipMemcpy(Sxy.data(), ctx->d_Sxy, sizeof(double) * nA, hipMemcpyDeviceToHost));
   auto get_list = [&](int n, const int32_t *drow, const int32_t *dptr, const int32_t *dcol,
                       std::vector<int32_t> &row, std::vector<int32_t> &ptr, std::vector<int32_t> &cl) -> int {
     row.resize(n);
@@ -2448,9 +2443,34 @@ static int amg_setup(ufe_ctx *ctx) {
     HIPCHK(ctx, hipMemcpy(cl.data(), dcol, sizeof(int32_t) * ptr[n], hipMemcpyDeviceToHost));
     return UFE_OK;
   };
-  std::vector<int32_t> nrow, nptr, ncol, crow, cptr2, ccol;
-  if ((r = get_list(ctx->n_neu, ctx->d_neu_row, ctx->d_neu_ptr, ctx->d_neu_col, nrow, nptr, ncol))) return r;
-  if ((r = get_list(ctx->n_cor, ctx->d_cor_row, ctx->d_cor_ptr, ctx->d_cor_col, crow, cptr2, ccol))) return r;
+  if ((r = get_list(ctx->n_neu, ctx->d_neu_row, ctx->d_neu_ptr, ctx->d_neu_col, L.nrow, L.nptr, L.ncol))) return r;
+  if ((r = get_list(ctx->n_cor, ctx->d_cor_row, ctx->d_cor_ptr, ctx->d_cor_col, L.crow, L.cptr2, L.ccol))) return r;
+  L.deg.resize(nA);
+  HIPCHK(ctx, hipMemcpy(L.deg.data(), ctx->d_deg, nA, hipMemcpyDeviceToHost));
+  std::vector<int64_t> cptr(nchunk + 1);
+  HIPCHK(ctx, hipMemcpy(cptr.data(), ctx->d_chunk_ptr, sizeof(int64_t) * (nchunk + 1), hipMemcpyDeviceToHost));
+  L.col.resize(cptr[nchunk]);
+  HIPCHK(ctx, hipMemcpy(L.col.data(), ctx->d_col, sizeof(int32_t) * L.col.size(), hipMemcpyDeviceToHost));
+  L.cptr = std::move(cptr);          // last: marks the lists as read
+  return UFE_OK;
+}
+
+static int amg_setup(ufe_ctx *ctx, HostLists &H) {
+  if (ctx->amg_ready) return UFE_OK;
+  const auto t0 = std::chrono::steady_clock::now();
+  const int nA = ctx->nA;
+  int r;
+  // the fine operator, read back from the device
+  if ((r = host_lists(ctx, H))) return r;
+  const std::vector<int64_t> &cptr = H.cptr;
+  const std::vector<uint8_t> &deg = H.deg;
+  const std::vector<int32_t> &col = H.col, &nrow = H.nrow, &nptr = H.nptr, &ncol = H.ncol, &crow = H.crow,
+                             &cptr2 = H.cptr2, &ccol = H.ccol;
+  const int64_t ne = (int64_t)col.size();
+  std::vector<double2> cU(ne);
+  std::vector<double> Sxy(nA);
+  HIPCHK(ctx, hipMemcpy(cU.data(), ctx->d_cU, sizeof(double2) * ne, hipMemcpyDeviceToHost));
+  HIPCHK(ctx, hipMemcpy(Sxy.data(), ctx->d_Sxy, sizeof(double) * nA, hipMemcpyDeviceToHost));
   // fine points: the SOR rows in colour order
   std::vector<int32_t> pid(nA, -1), rows;
   for (int c = 0; c < 5; c++)
@@ -2973,44 +2993,53 @@ static int patch_alloc(ufe_ctx *ctx, T *&p, size_t n) {
   return UFE_OK;
 }
 
-// The parts of one patch set, joined by the host's threads and copied to one device
-// allocation at once (S.P.d null: no room); a copy for each of nine arrays of 16
-// parts took longer than the walk.
-static int patch_upload(ufe_ctx *ctx, const std::vector<PatchHost> &parts, PatchSet &S) {
-  auto fields = [&](auto f) {
-    f(0, &PatchHost::d, S.P.d);
-    f(1, &PatchHost::rows, S.P.rows);
-    f(2, &PatchHost::nptr, S.P.nptr);
-    f(3, &PatchHost::sbase, S.P.sbase);
-    f(4, &PatchHost::lcol, S.P.lcol);
-    f(5, &PatchHost::ov_e, S.P.ov_e);
-    f(6, &PatchHost::ovf, S.P.ovf);
-    f(7, &PatchHost::ov_c, S.P.ov_c);
-    f(8, &PatchHost::ncol, S.P.ncol);
-  };
+// One patch set as it goes to the device: its nine arrays, each of all parts, in one
+// piece (a copy for each array of 16 parts took longer than the walk)
+struct PatchImage {
+  std::unique_ptr<char[]> host;
+  size_t total = 0, first[9];        // bytes, and where each array starts
+};
+extern "C++" template <typename F>
+static void patch_arrays(PatchDev &P, F f) {
+  f(0, &PatchHost::d, P.d);
+  f(1, &PatchHost::rows, P.rows);
+  f(2, &PatchHost::nptr, P.nptr);
+  f(3, &PatchHost::sbase, P.sbase);
+  f(4, &PatchHost::lcol, P.lcol);
+  f(5, &PatchHost::ov_e, P.ov_e);
+  f(6, &PatchHost::ovf, P.ovf);
+  f(7, &PatchHost::ov_c, P.ov_c);
+  f(8, &PatchHost::ncol, P.ncol);
+}
+static void patch_pack(std::vector<PatchHost> &parts, int threads, PatchImage &I) {
   std::vector<size_t> first[9];      // of each array: the first byte of each part
-  size_t total = 0;
-  fields([&](int k, auto field, auto *&dst) {
-    first[k].assign(1, total);
-    for (const PatchHost &H : parts) first[k].push_back(first[k].back() + (H.*field).size() * sizeof(*dst));
-    total = (first[k].back() + 255) / 256 * 256;
+  PatchDev P{};
+  I.total = 0;
+  patch_arrays(P, [&](int k, auto field, auto *&p) {
+    first[k].assign(1, I.first[k] = I.total);
+    for (const PatchHost &H : parts) first[k].push_back(first[k].back() + (H.*field).size() * sizeof(*p));
+    I.total = (first[k].back() + 255) / 256 * 256;
   });
-  char *base = nullptr;
-  if (const int r = patch_alloc(ctx, base, total)) return r;
-  if (!base) return UFE_OK;
-  const std::unique_ptr<char[]> host(new char[total]);
-  const int threads = (int)std::min({parts.size(), (size_t)patch_threads(ctx->nA), 1 + (total >> 20)});
-  amg_parts((int)parts.size(), threads, [&](int, int t0, int t1) {
-    for (int t = t0; t < t1; t++)
-      fields([&](int k, auto field, auto *&) {
+  I.host.reset(new char[I.total]);
+  const int n = (int)parts.size();
+  amg_parts(n, (int)std::min<size_t>(std::min(n, threads), 1 + (I.total >> 20)), [&](int, int t0, int t1) {
+    for (int t = t0; t < t1; t++) {
+      patch_arrays(P, [&](int k, auto field, auto *&) {
         const auto &v = parts[t].*field;
-        if (!v.empty()) std::memcpy(host.get() + first[k][t], v.data(), first[k][t + 1] - first[k][t]);
+        if (!v.empty()) std::memcpy(I.host.get() + first[k][t], v.data(), first[k][t + 1] - first[k][t]);
       });
+      parts[t] = PatchHost{};
+    }
   });
-  HIPCHK(ctx, hipMemcpyAsync(base, host.get(), total, hipMemcpyHostToDevice, ctx->stream));
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));   // the host copy goes with this call
-  fields([&](int k, auto, auto *&dst) {
-    dst = reinterpret_cast<std::remove_reference_t<decltype(dst)>>(base + first[k][0]);
+}
+static int patch_upload(ufe_ctx *ctx, const PatchImage &I, PatchSet &S) {   // S.P.d null: no room
+  char *base = nullptr;
+  if (const int r = patch_alloc(ctx, base, I.total)) return r;
+  if (!base) return UFE_OK;
+  HIPCHK(ctx, hipMemcpyAsync(base, I.host.get(), I.total, hipMemcpyHostToDevice, ctx->stream));
+  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));   // the image goes with the caller
+  patch_arrays(S.P, [&](int k, auto, auto *&p) {
+    p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(base + I.first[k]);
   });
   return UFE_OK;
 }
@@ -3049,83 +3078,99 @@ static void patch_find(const ufe_ctx *ctx, const PatchMesh &m, const std::vector
   if (fits && sor) patch_mark_shared(ctx->nA, parts);
 }
 
-// Builds the wanted patch sets that are not there yet
+// Builds the wanted patch sets that are not there yet: start() walks them on host
+// threads of its own, side by side, and finish() takes them to the device, so that a
+// multigrid set-up runs meanwhile.  The lists and the context's mesh outlive it.
 static bool sor_patch_resident(ufe_ctx *ctx, const PatchSet &S);
-static int patch_prepare(ufe_ctx *ctx, std::initializer_list<PatchKind> kinds, int nu) try {
-  bool all = true;
-  for (PatchKind k : kinds) all = all && ctx->patch[k][nu - 1].built;
-  if (all) return UFE_OK;
-  const int nA = ctx->nA, nchunk = (nA + SELL - 1) / SELL;
-  std::vector<int64_t> cptr(nchunk + 1);
-  std::vector<uint8_t> deg(nA);
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  HIPCHK(ctx, hipMemcpy(cptr.data(), ctx->d_chunk_ptr, sizeof(int64_t) * (nchunk + 1), hipMemcpyDeviceToHost));
-  HIPCHK(ctx, hipMemcpy(deg.data(), ctx->d_deg, nA, hipMemcpyDeviceToHost));
-  std::vector<int32_t> col(cptr[nchunk]);
-  HIPCHK(ctx, hipMemcpy(col.data(), ctx->d_col, sizeof(int32_t) * col.size(), hipMemcpyDeviceToHost));
-  auto get = [&](int n, const int32_t *dp, std::vector<int32_t> &h) -> int {
-    h.resize(std::max(n, 1));
-    if (n) HIPCHK(ctx, hipMemcpy(h.data(), dp, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
+class PatchWalk {
+ public:
+  PatchWalk(ufe_ctx *c, HostLists &l) : ctx(c), L(l) {}
+  ~PatchWalk() { join(); }
+  int start(std::initializer_list<PatchKind> kinds, int sweeps) {
+    nu = sweeps;
+    for (PatchKind k : kinds)
+      if (!ctx->patch[k][nu - 1].built) todo.push_back(k);
+    if (todo.empty()) return UFE_OK;
+    if (const int r = host_lists(ctx, L)) return r;
+    set.resize(todo.size());
+    image.resize(todo.size());
+    try {
+      th = std::thread([this] { walk(); });
+    } catch (const std::exception &) {
+      walk();
+    }
     return UFE_OK;
-  };
-  int r;
-  std::vector<int32_t> nr, np, nc, kr, kp, kc;
-  if ((r = get(ctx->n_neu, ctx->d_neu_row, nr)) || (r = get(ctx->n_neu + 1, ctx->d_neu_ptr, np)) ||
-      (r = get(np[ctx->n_neu], ctx->d_neu_col, nc)) || (r = get(ctx->n_cor, ctx->d_cor_row, kr)) ||
-      (r = get(ctx->n_cor + 1, ctx->d_cor_ptr, kp)) || (r = get(kp[ctx->n_cor], ctx->d_cor_col, kc)))
-    return r;
-  const PatchMesh m{nA, ctx->colour_start, ctx->colour_active, cptr.data(), deg.data(), col.data(), ctx->n_neu,
-                    ctx->n_cor, nr.data(), np.data(), nc.data(), kr.data(), kp.data(), kc.data(), ctx->h_key.data(),
-                    ctx->h_mid.empty() ? nullptr : ctx->h_mid.data()};
-  const std::vector<int32_t> order = patch_order(m);
-  if (!ctx->d_place) {
-    std::vector<int32_t> place(nA, 0);
-    for (int i = 0; i < ctx->n_neu; i++) place[nr[i]] = i + 1;
-    for (int i = 0; i < ctx->n_cor; i++) place[kr[i]] = -i - 1;
-    std::vector<int32_t> met(kr.begin(), kr.begin() + ctx->n_cor);
-    met.insert(met.end(), kc.begin(), kc.begin() + kp[ctx->n_cor]);
-    std::sort(met.begin(), met.end());
-    ctx->cor_apart = std::adjacent_find(met.begin(), met.end()) == met.end();
-    int32_t *d_place = nullptr;
-    if ((r = patch_alloc(ctx, d_place, (size_t)nA))) return r;
-    if (d_place) HIPCHK(ctx, hipMemcpy(d_place, place.data(), sizeof(int32_t) * nA, hipMemcpyHostToDevice));
-    ctx->d_place = d_place;
   }
-  // the sets are walked side by side, each by its share of the threads
-  std::vector<PatchKind> todo;
-  for (PatchKind k : kinds)
-    if (!ctx->patch[k][nu - 1].built) todo.push_back(k);
-  std::vector<std::vector<PatchHost>> parts(todo.size());
-  const int threads = patch_threads(nA), nk = (int)todo.size(), each = std::max(1, threads / nk);
-  amg_parts(nk, std::min(nk, threads), [&](int, int i0, int i1) {
-    for (int i = i0; i < i1; i++) {
-      PatchSet &S = ctx->patch[todo[i]][nu - 1];
-      try {
-        patch_find(ctx, m, order, todo[i], nu, each, parts[i], S);
-      } catch (const std::bad_alloc &) {
-        S.bs = 0;
+  int finish() {
+    join();
+    if (todo.empty()) return UFE_OK;
+    int r;
+    if (!ctx->d_place && !place.empty()) {
+      int32_t *d = nullptr;
+      if ((r = patch_alloc(ctx, d, place.size()))) return r;
+      if (d) HIPCHK(ctx, hipMemcpy(d, place.data(), sizeof(int32_t) * place.size(), hipMemcpyHostToDevice));
+      ctx->cor_apart = apart;
+      ctx->d_place = d;
+    }
+    for (size_t i = 0; i < todo.size(); i++) {
+      PatchSet &S = set[i];
+      ctx->paths.patch_sets++;
+      if (S.bs) {
+        if ((r = patch_upload(ctx, image[i], S))) return r;
+        S.ok = S.P.d && (todo[i] != PATCH_SOR64 || sor_patch_resident(ctx, S));
       }
+      S.built = true;
+      ctx->patch[todo[i]][nu - 1] = S;
     }
-  });
-  for (int i = 0; i < nk; i++) {
-    PatchSet &S = ctx->patch[todo[i]][nu - 1];
-    ctx->paths.patch_sets++;
-    if (S.bs) {
-      if ((r = patch_upload(ctx, parts[i], S))) return r;
-      S.ok = S.P.d && (todo[i] != PATCH_SOR64 || sor_patch_resident(ctx, S));
-    }
-    S.built = true;
+    return UFE_OK;
   }
-  return UFE_OK;
-} catch (const std::bad_alloc &) {   // no host memory: the colour launches do without
-  for (PatchKind k : kinds) ctx->patch[k][nu - 1].built = true;
-  return UFE_OK;
-}
+
+ private:
+  ufe_ctx *ctx;
+  HostLists &L;
+  int nu = 1;
+  std::vector<PatchKind> todo;
+  std::vector<PatchSet> set;         // bs 0: the mesh does not fit, or no host memory
+  std::vector<PatchImage> image;
+  std::vector<int32_t> place;
+  bool apart = false;
+  std::thread th;
+  void join() {
+    if (th.joinable()) th.join();
+  }
+  void walk() noexcept {
+    try {
+      const int nA = ctx->nA, nk = (int)todo.size(), threads = patch_threads(nA), each = std::max(1, threads / nk);
+      const PatchMesh m{nA, ctx->colour_start, ctx->colour_active, L.cptr.data(), L.deg.data(), L.col.data(), ctx->n_neu,
+                        ctx->n_cor, L.nrow.data(), L.nptr.data(), L.ncol.data(), L.crow.data(), L.cptr2.data(),
+                        L.ccol.data(), ctx->h_key.data(), ctx->h_mid.empty() ? nullptr : ctx->h_mid.data()};
+      const std::vector<int32_t> order = patch_order(m);
+      amg_parts(nk, std::min(nk, threads), [&](int, int i0, int i1) {
+        for (int i = i0; i < i1; i++) try {
+            std::vector<PatchHost> parts;
+            patch_find(ctx, m, order, todo[i], nu, each, parts, set[i]);
+            if (set[i].bs) patch_pack(parts, each, image[i]);
+          } catch (const std::bad_alloc &) {   // the colour launches do without
+            set[i].bs = 0;
+          }
+      });
+      std::vector<int32_t> at(nA, 0), met(L.crow);
+      for (int i = 0; i < ctx->n_neu; i++) at[L.nrow[i]] = i + 1;
+      for (int i = 0; i < ctx->n_cor; i++) at[L.crow[i]] = -i - 1;
+      met.insert(met.end(), L.ccol.begin(), L.ccol.end());
+      std::sort(met.begin(), met.end());
+      apart = std::adjacent_find(met.begin(), met.end()) == met.end();
+      place = std::move(at);
+    } catch (const std::exception &) {
+      for (PatchSet &S : set) S.bs = 0;
+    }
+  }
+};
 
 // The smoothing of the multigrid cycle runs on patches (one or two sweeps; the
 // per-colour kernels otherwise, or with UFE_AMG_PATCH=0 in the environment when
 // the hierarchy is first used with this sweep count).
-static int amg_patches(ufe_ctx *ctx) {
+static int amg_patches_start(ufe_ctx *ctx, PatchWalk &walk) {
   const int nu = std::max(1, ctx->amg_nu);
   if (nu > 2) return UFE_OK;
   const char *off = std::getenv("UFE_AMG_PATCH");
@@ -3133,8 +3178,16 @@ static int amg_patches(ufe_ctx *ctx) {
     for (PatchKind k : {PATCH_PRE32, PATCH_POST32}) ctx->patch[k][nu - 1].built = true;
     return UFE_OK;
   }
+  return walk.start({PATCH_PRE32, PATCH_POST32}, nu);
+}
+// The hierarchy (ctx->amg_nu set) and, meanwhile, the patches of the fine smoothing
+static int amg_prepare(ufe_ctx *ctx) {
+  HostLists lists;
+  PatchWalk walk(ctx, lists);
   int r;
-  if ((r = patch_prepare(ctx, {PATCH_PRE32, PATCH_POST32}, nu))) return r;
+  if ((r = amg_patches_start(ctx, walk)) || (r = amg_setup(ctx, lists)) || (r = walk.finish())) return r;
+  const int nu = std::max(1, ctx->amg_nu);
+  if (nu > 2 || !ctx->patch[PATCH_PRE32][nu - 1].ok || !ctx->patch[PATCH_POST32][nu - 1].ok) return UFE_OK;
   return patch_spaces([&](auto *&p) { return patch_alloc(ctx, p, (size_t)ctx->nA); }, ctx->amg_zt, ctx->amg_zu);
 }
 static bool amg_on_patches(const ufe_ctx *ctx) {
@@ -3477,7 +3530,9 @@ static const PatchSet *sor_patches(ufe_ctx *ctx, int *err) {
       S.built = true;
       return nullptr;
     }
-    if ((*err = patch_prepare(ctx, {PATCH_SOR64}, 1))) return nullptr;
+    HostLists lists;
+    PatchWalk walk(ctx, lists);
+    if ((*err = walk.start({PATCH_SOR64}, 1)) || (*err = walk.finish())) return nullptr;
   }
   if (S.ok && !ctx->sor_ready) {
     if ((*err = sor_spaces(ctx))) return nullptr;
@@ -4162,8 +4217,7 @@ int ufe_ssa_linear_solve(ufe_ctx *ctx, const ufe_linsolve_opts *o, ufe_linsolve_
   }
   if (ctx->pc_amg) {
     ctx->amg_T = false;
-    if ((r = amg_setup(ctx))) return r;
-    if ((r = amg_patches(ctx))) return r;
+    if ((r = amg_prepare(ctx))) return r;
     amg_refresh(ctx);
     LAUNCHCHK(ctx);
     if ((r = amg_capture(ctx))) return r;
@@ -4431,9 +4485,8 @@ static int adj_solve(ufe_ctx *ctx, double tol, int m, int ks, double omega, int 
   if (mg) {                           // the transposed hierarchy for this system's diagonals
     int r;
     ctx->amg_T = false;
-    if ((r = amg_setup(ctx))) return r;
     ctx->amg_nu = ks;
-    if ((r = amg_patches(ctx))) return r;
+    if ((r = amg_prepare(ctx))) return r;
     const char *fold = std::getenv("UFE_FOLD_MAX");
     ctx->fold_max = fold && *fold ? (int)std::strtol(fold, nullptr, 10) : FOLD_MAX;
     if (amg_on_patches(ctx) && !ctx->amg_zt64 && (r = patch_alloc(ctx, ctx->amg_zt64, (size_t)n))) return r;
@@ -4881,8 +4934,7 @@ int ufe_batch_linear_solve(ufe_ctx *ctx, const ufe_batch_opts *o, double *member
   if (f32) k_to_f32_pair<<<nblk(ctx->nA), BLOCK, 0, ctx->stream>>>(ctx->nA, ctx->d_pair[1], ctx->d_EV32);
   if (ctx->pc_amg) {                  // the union of the members as one hierarchy
     ctx->amg_T = false;
-    if ((r = amg_setup(ctx))) return r;
-    if ((r = amg_patches(ctx))) return r;
+    if ((r = amg_prepare(ctx))) return r;
     amg_refresh(ctx);
     LAUNCHCHK(ctx);
     if ((r = amg_capture(ctx))) return r;
