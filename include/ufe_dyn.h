@@ -228,7 +228,7 @@ typedef struct ufe_linsolve_stats {
 } ufe_linsolve_stats;
 
 /* Live kernel timing: start/stop events attached to the dispatch of every
- * 8th SOR colour-kernel launch (hipExtLaunchKernelGGL), i.e. the kernel's own
+ * 7th SOR colour-kernel launch (hipExtLaunchKernelGGL), i.e. the kernel's own
  * execution time on the library's stream.  Where the multigrid smoothing runs on
  * patches, its launches count instead: all sweeps of a smoothing in one, with the
  * bytes that one launch needs (each input once). */

@@ -252,3 +252,27 @@ def test_adjoint_folds_in_one_launch_and_in_several(gl):
     for name in ("one", "several"):
         for a, b in zip(out["colours"], out[name]):
             assert torch.equal(a, b) and float(a.abs().max()) > 0, name
+
+
+def test_profile_samples_both_smoothings():
+    """The two smoothings of an application alternate and differ in bytes and time:
+    the sampled mean lies between theirs."""
+    print("[patch profile] both", flush=True)
+    wl = geometry.marine(6000, seed=5, picard=2)
+    ctx = abi.Context(0)
+    try:
+        frozen_ssa_system(ctx, wl, picard=2)
+        ctx.profile_read()
+        ctx.profile_enable(True)
+        for _ in range(3):
+            ctx.ssa_linear_solve(1e-8, 1000, precision=abi.UFE_MIXED, gmres=20, precond_sweeps=2, orth_passes=1,
+                                 precond_type=abi.UFE_PRECOND_MULTIGRID)
+        ctx.profile_enable(False)
+        p, sweep = ctx.profile_read(), ctx.sweep_bytes()
+        assert p.launches >= 8 and p.total_launches >= 7 * (p.launches - 1)
+        pre = (10.0 * sweep["mean_degree"] + 44.0) * sweep["rows"]       # coefficients, columns, row data, z and residual
+        post = pre + 8.0 * sweep["rows"]                                 # and the values it starts from
+        mean = p.algorithmic_bytes / p.launches
+        assert pre + 0.3 * (post - pre) < mean < pre + 0.7 * (post - pre), (pre, mean, post)
+    finally:
+        ctx.close()

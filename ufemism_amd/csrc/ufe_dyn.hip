@@ -366,7 +366,9 @@ static uint64_t hilbert_index(uint32_t x, uint32_t y) {
 }
 
 static inline int nblk(int64_t n, int b = BLOCK) { return (int)((n + b - 1) / b); }
-constexpr int PROF_EVERY = 8;     // colour launches per timed sample
+// launches per timed sample: odd and no multiple of five, so that the sample goes
+// through both smoothings of an application and all colours
+constexpr int PROF_EVERY = 7;
 // grid for XCD-major kernels: a multiple of the 8 XCDs
 static inline int xcd_grid(int64_t n) { return (nblk(n) + 7) / 8 * 8; }
 // grid of a layered kernel: points, groups of G layers, fields
