@@ -457,7 +457,8 @@ int ufe_ssa_adjoint_backward(ufe_ctx *ctx, const double *dJ_dU, const double *dJ
  * flight, 3: plain loads, all six slots' loads of a six-slot row in one batch).
  * All give identical results.  The autotuner times `sweeps` sweeps
  * of the uploaded mesh (single or batch) per shape and keeps the fastest for
- * every later FP32 sweep of the context (default: 256, 0, 0). */
+ * every later FP32 colour launch of the context (default: 256, 0, 0); one or two
+ * multigrid smoothing sweeps run on patches, which have shapes of their own. */
 typedef struct ufe_sweep_tuning {
   int32_t threads_per_block;
   int32_t schedule;
