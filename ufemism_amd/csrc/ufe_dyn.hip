@@ -5231,7 +5231,8 @@ int ufe_op_neumann_AaAc(ufe_ctx *ctx, double *d) {
   NEED_MESH(ctx);
   if (ctx->n_neu)
     k_neumann_scalar<<<nblk(ctx->n_neu), BLOCK, 0, ctx->stream>>>(neu_list(ctx), ctx->d_perm, d);
-  k_neumann_scalar<<<nblk(ctx->n_cor, 64), 64, 0, ctx->stream>>>(cor_list(ctx), ctx->d_perm, d);
+  if (ctx->n_cor)                    // a batch need not have corner codes
+    k_neumann_scalar<<<nblk(ctx->n_cor, 64), 64, 0, ctx->stream>>>(cor_list(ctx), ctx->d_perm, d);
   LAUNCHCHK(ctx);
   return ufe_synchronize(ctx);
 }
